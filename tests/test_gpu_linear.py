@@ -119,3 +119,34 @@ def test_linear_quadrant_tiles(reef, rows, fout, quadrants, monkeypatch):
     y = host(reef.linear_w8a8(gpu(x), gpu(w), gpu(ws), gpu(b)))
     gold = oracle_linear(x, w, ws, b)
     assert np.array_equal(y.view(np.uint32), gold.view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,fin,fout", [
+    (1, 16, 1), (16, 528, 301), (31, 1040, 513),   # 16 features, one or more blocks of 16 rows
+    (17, 144, 4001),                               # 16 features, 32 rows
+    (16, 272, 6101), (3, 2064, 6100),              # 32 features, 16 rows
+    (100, 400, 2101), (65, 1040, 4160),            # 64 x 64 tiles
+    (300, 272, 5001),                              # 128 x 64
+    (520, 128, 6500),                              # 128 x 128
+    (4000, 160, 1270),                             # 128 x 160
+    (2001, 400, 4002),                             # 256 x 128
+    (2040, 144, 6101),                             # 256 x 192
+    (4090, 272, 4095),                             # 256 x 256
+])
+def test_linear_every_kernel_bit_exact(reef, rows, fin, fout):
+    """One shape for each kernel and tile that the launch chooses between on 256 compute
+    units, with partial tiles at both edges, K steps that end inside a 128-byte step,
+    fewer steps than LDS stages, and rows of y that are not 16-byte aligned."""
+    case(f"w8a8 kernels rows{rows} in{fin} out{fout}")
+    rng = np.random.default_rng(rows + fin + fout)
+    x = rng.standard_normal((rows, fin), dtype=np.float32)
+    w = rng.integers(-127, 128, (fout, fin), dtype=np.int8)
+    ws = rng.uniform(0.001, 0.02, fout).astype(np.float32)
+    b = rng.standard_normal(fout).astype(np.float32)
+    y = host(reef.linear_w8a8(gpu(x), gpu(w), gpu(ws), gpu(b)))
+    q, s = oracle.quantize_rows(x)
+    # integer sums below 2^53 are exact in float64
+    acc = (q.astype(np.float64) @ w.astype(np.float64).T).astype(np.float32)
+    gold = acc * (s[:, None] * ws[None, :]) + b[None, :]
+    assert gold.dtype == np.float32
+    assert np.array_equal(y.view(np.uint32), gold.view(np.uint32))
