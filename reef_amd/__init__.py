@@ -17,6 +17,7 @@ from __future__ import annotations
 import ctypes as C
 import math
 import os
+import struct
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(PKG, "libreef_hip.so")
@@ -102,44 +103,39 @@ class KvAppendParams(C.Structure):
 
 _P = C.c_void_p
 _I64 = C.c_int64
+_S = C.c_void_p  # a structure: byref(...) or its bytes
 _SIGS = {
     "reef_quantize_int8_per_tensor": [_P, _I64, _P, _P, _P, _P],
-    "reef_quantize_int8_per_head": [_P, _I64, _I64, _I64, _I64, C.POINTER(Strides), _P, _P, _P,
-                                    _P],
+    "reef_quantize_int8_per_head": [_P, _I64, _I64, _I64, _I64, _S, _P, _P, _P, _P],
     "reef_quantize_int8_per_token": [_P, _I64, _I64, _I64, _P, _P, _P, _P],
     "reef_dequantize_int8": [_P, _I64, _I64, _P, _P, _P],
     "reef_read_status_word": [_P, C.c_int, _P],
-    "reef_attention_prefill_workspace_bytes": [C.POINTER(AttentionParams)],
-    "reef_attention_prefill_int8": [C.POINTER(AttentionParams), _P, C.POINTER(Strides), _P,
-                                    C.POINTER(Strides), _P, C.POINTER(Strides), _P, _P, _P, _P,
-                                    C.POINTER(Strides), _P, C.c_size_t, _P],
+    "reef_attention_prefill_workspace_bytes": [_S],
+    "reef_attention_prefill_int8": [_S, _P, _S, _P, _S, _P, _S, _P, _P, _P, _P, _S, _P,
+                                    C.c_size_t, _P],
     "reef_qk_scores_i32": [_P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P],
     "reef_qk_scores_i32_packed_workspace_bytes": [_I64, _I64, _I64, _I64, _I64],
     "reef_qk_scores_i32_packed": [_P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, C.c_size_t, _P],
-    "reef_attention_decode_workspace_bytes": [C.POINTER(DecodeParams)],
-    "reef_attention_decode_int8": [C.POINTER(DecodeParams), _P, _P, _P, _P, _P, _P, _P, _P, _P,
-                                   C.c_size_t, _P, _P],
-    "reef_attention_decode_int8_paged": [C.POINTER(DecodeParams), _P, _P, _P, _P, _P, _P, _P,
+    "reef_attention_decode_workspace_bytes": [_S],
+    "reef_attention_decode_int8": [_S, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P,
+                                   _P],
+    "reef_attention_decode_int8_paged": [_S, _P, _P, _P, _P, _P, _P, _P,
                                          _I64, _I64, _P, _P, _P, C.c_size_t, _P, _P],
-    "reef_attention_decode_int8_paged_noalloc": [C.POINTER(DecodeParams), _P, _P, _P, _P, _P, _P,
+    "reef_attention_decode_int8_paged_noalloc": [_S, _P, _P, _P, _P, _P, _P,
                                                  _P, _I64, _I64, _P, _P, _P, _P],
     "reef_kv_pack_v_pages": [_P, _I64, _I64, _P, _P],
     "reef_linear_w8a8_workspace_bytes": [_I64, _I64],
     "reef_linear_w8a8": [_P, _I64, _I64, _I64, _P, _P, _P, _I64, _P, _I64, _P, C.c_size_t, _P,
                          _P],
     "reef_gemm_w8a8": [_P, _P, _I64, _I64, _P, _P, _P, _I64, _P, _I64, _P, _P],
-    "reef_attention_int8_integer": [C.POINTER(AttentionParams), _P, C.POINTER(Strides), _P,
-                                    C.POINTER(Strides), _P, C.POINTER(Strides), C.c_uint32, _P,
-                                    C.c_uint32, _P, C.POINTER(Strides), _P],
-    "reef_kv_append_int8": [C.POINTER(KvAppendParams), _P, C.POINTER(Strides), _P,
-                            C.POINTER(Strides), _P, _P, _P, _P, _P, _P, _P, _P],
-    "reef_kv_append_int8_paged": [C.POINTER(KvAppendParams), _P, C.POINTER(Strides), _P,
-                                  C.POINTER(Strides), _P, _P, _I64, _I64, _P, _P, _P, _P, _P,
-                                  _P, _P],
-    "reef_attention_prefill_cache_workspace_bytes": [C.POINTER(AttentionParams)],
-    "reef_attention_prefill_int8_cache": [C.POINTER(AttentionParams), _P, C.POINTER(Strides), _P,
-                                          _P, _P, _P, _P, _I64, _P, _I64, _I64, _P,
-                                          C.POINTER(Strides), _P, C.c_size_t, _P, _P],
+    "reef_attention_int8_integer": [_S, _P, _S, _P, _S, _P, _S, C.c_uint32, _P, C.c_uint32, _P,
+                                    _S, _P],
+    "reef_kv_append_int8": [_S, _P, _S, _P, _S, _P, _P, _P, _P, _P, _P, _P, _P],
+    "reef_kv_append_int8_paged": [_S, _P, _S, _P, _S, _P, _P, _I64, _I64, _P, _P, _P, _P, _P, _P,
+                                  _P],
+    "reef_attention_prefill_cache_workspace_bytes": [_S],
+    "reef_attention_prefill_int8_cache": [_S, _P, _S, _P, _P, _P, _P, _P, _I64, _P, _I64, _I64,
+                                          _P, _S, _P, C.c_size_t, _P, _P],
 }
 
 _lib_handle = None
@@ -167,32 +163,65 @@ def check(status: int, what: str) -> None:
 
 # --- torch plumbing -------------------------------------------------------------------
 
+# The wrappers below run once per layer and token of a serving loop, so the small calls are
+# bound by this file: arguments go to the library as plain addresses and packed bytes
+# (a ctypes structure costs four times its bytes), and the stream is read as a handle
+# rather than through a torch.cuda.Stream (a 1x1x128x64 prefill: 11.4 us a call against
+# 20.5, of which 8 us are the kernel's).
+
+_torch_module = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        _torch_module = torch
+    return _torch_module
 
 
 def _stream():
-    return C.c_void_p(_torch().cuda.current_stream().cuda_stream)
+    """The current device's current stream, as an address."""
+    c = _torch()._C
+    try:
+        return c._cuda_getCurrentRawStream(c._cuda_getDevice())
+    except AttributeError:
+        return _torch().cuda.current_stream().cuda_stream
 
 
 def _ptr(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
+
+
+def _packed(layout, structure, *fields):
+    """The bytes of `structure` (whose members `layout` gives) for the library to read."""
+    try:
+        return layout.pack(*fields)
+    except (struct.error, OverflowError):  # a value outside its member's range
+        return C.byref(structure(*fields))
+
+
+_STRIDES = struct.Struct("=3q")
+_ATTENTION = struct.Struct("=8qf2iI")
+_DECODE = struct.Struct("=6qf2iI")
+_APPEND = struct.Struct("=5q")
 
 
 def _require(t, dtype, name):
     torch = _torch()
-    if not isinstance(t, torch.Tensor) or not t.is_cuda:
-        raise InvalidArgument(f"{name} must be a GPU tensor")
-    if t.dtype != dtype:
+    if isinstance(t, torch.Tensor) and t.is_cuda:
+        if t.dtype == dtype:
+            return
         raise InvalidArgument(f"{name} must be {dtype}, got {t.dtype}")
+    raise InvalidArgument(f"{name} must be a GPU tensor")
 
 
 def _strides4(t):
     """Strides of a [B, H, S, D] tensor with a contiguous last dimension."""
-    if t.dim() != 4 or t.stride(3) != 1:
+    st = t.stride()
+    if len(st) != 4 or st[3] != 1:
         raise InvalidArgument("expected [batch, heads, tokens, head_dim] with contiguous head_dim")
-    return Strides(t.stride(0), t.stride(1), t.stride(2))
+    return _STRIDES.pack(st[0], st[1], st[2])
 
 
 class StatusWord:
@@ -204,7 +233,7 @@ class StatusWord:
 
     @property
     def ptr(self):
-        return _ptr(self.tensor)
+        return C.c_void_p(self.tensor.data_ptr())
 
     def check(self, what: str) -> None:
         check(lib().reef_read_status_word(self.ptr, 1, _stream()), what)
@@ -220,7 +249,7 @@ def quantize_per_tensor(x, status: StatusWord | None = None):
     q = torch.empty(x.shape, dtype=torch.int8, device=x.device)
     s = torch.empty(1, dtype=torch.float32, device=x.device)
     own = status or StatusWord(x.device)
-    check(lib().reef_quantize_int8_per_tensor(_ptr(x), x.numel(), _ptr(q), _ptr(s), own.ptr,
+    check(lib().reef_quantize_int8_per_tensor(_ptr(x), x.numel(), _ptr(q), _ptr(s), _ptr(own.tensor),
                                               _stream()), "quantize_per_tensor")
     if status is None:
         own.check("quantize_per_tensor requires finite values")
@@ -237,8 +266,8 @@ def quantize_per_head(x, status: StatusWord | None = None):
     q = torch.empty((B, H, S, D), dtype=torch.int8, device=x.device)
     s = torch.empty(H, dtype=torch.float32, device=x.device)
     own = status or StatusWord(x.device)
-    check(lib().reef_quantize_int8_per_head(_ptr(x), B, H, S, D, C.byref(st), _ptr(q), _ptr(s),
-                                            own.ptr, _stream()), "quantize_per_head")
+    check(lib().reef_quantize_int8_per_head(_ptr(x), B, H, S, D, st, _ptr(q), _ptr(s),
+                                            _ptr(own.tensor), _stream()), "quantize_per_head")
     if status is None:
         own.check("quantize_per_head requires finite values")
     return q, s
@@ -249,19 +278,20 @@ def quantize_rows(x, status: StatusWord | None = None):
     (per token). Returns int8 of x's shape and scales of x.shape[:-1]."""
     torch = _torch()
     _require(x, torch.float32, "x")
-    width = x.shape[-1]
-    x2 = x.reshape(-1, width)
+    shape = x.shape
+    width = shape[-1]
+    x2 = x if len(shape) == 2 else x.reshape(-1, width)
     if x2.stride(1) != 1:
         x2 = x2.contiguous()
     rows = x2.shape[0]
-    q = torch.empty((rows, width), dtype=torch.int8, device=x.device)
-    s = torch.empty(rows, dtype=torch.float32, device=x.device)
+    q = torch.empty(shape, dtype=torch.int8, device=x.device)
+    s = torch.empty(shape[:-1], dtype=torch.float32, device=x.device)
     own = status or StatusWord(x.device)
     check(lib().reef_quantize_int8_per_token(_ptr(x2), rows, width, x2.stride(0), _ptr(q),
-                                             _ptr(s), own.ptr, _stream()), "quantize_rows")
+                                             _ptr(s), _ptr(own.tensor), _stream()), "quantize_rows")
     if status is None:
         own.check("quantize_rows requires finite values")
-    return q.reshape(x.shape), s.reshape(x.shape[:-1])
+    return q, s
 
 
 quantize_per_token = quantize_rows
@@ -274,8 +304,9 @@ def dequantize(q, scales, group: int):
     _require(scales, torch.float32, "scales")
     q = q.contiguous()
     x = torch.empty(q.shape, dtype=torch.float32, device=q.device)
-    check(lib().reef_dequantize_int8(_ptr(q), q.numel(), group, _ptr(scales.contiguous()),
-                                     _ptr(x), _stream()), "dequantize")
+    scales = scales.contiguous()
+    check(lib().reef_dequantize_int8(_ptr(q), q.numel(), group, _ptr(scales), _ptr(x),
+                                     _stream()), "dequantize")
     return x
 
 
@@ -288,11 +319,15 @@ def prefill_workspace(params: AttentionParams, device):
     """The zero-filled workspace of the balanced prefill schedule, one per (device,
     stream): every launch leaves it zero-filled, so the next launch on that stream
     reuses it."""
-    torch = _torch()
-    n = lib().reef_attention_prefill_workspace_bytes(C.byref(params))
-    key = (torch.device(device).index, _stream().value)
+    return _prefill_workspace(C.byref(params), _torch().device(device), _stream())
+
+
+def _prefill_workspace(params, device, stream):
+    n = lib().reef_attention_prefill_workspace_bytes(params)
+    key = (device.index, stream)
     ws = _PREFILL_WS.get(key)
     if ws is None or ws.numel() < n:
+        torch = _torch()
         ws = torch.zeros(max(n, 256), dtype=torch.uint8, device=device)
         _PREFILL_WS[key] = ws
     return ws
@@ -322,19 +357,23 @@ def attention_prefill(q, k, v, q_scales, k_scales, v_scales, *, query_start=None
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
     start = Skv - Sq if query_start is None else query_start
-    p = AttentionParams(B, Hq, Hkv, Sq, Skv, D, start, window, softmax_scale, q_granularity,
-                        kv_granularity, (ATTN_PRECISE_PV if precise else 0) | schedule)
+    p = _packed(_ATTENTION, AttentionParams, B, Hq, Hkv, Sq, Skv, D, start, window, softmax_scale,
+                q_granularity, kv_granularity, (ATTN_PRECISE_PV if precise else 0) | schedule)
+    device = q.device
     if out is None:
-        out = torch.empty((B, Hq, Sq, D), dtype=torch.float32, device=q.device)
+        out = torch.empty((B, Hq, Sq, D), dtype=torch.float32, device=device)
     qs, ks, vs, os_ = _strides4(q), _strides4(k), _strides4(v), _strides4(out)
+    stream = _stream()
     if workspace is None:
-        workspace = prefill_workspace(p, q.device)
+        workspace = _prefill_workspace(p, device, stream)
     ws_ptr, ws_n = (None, 0) if workspace is False else (_ptr(workspace), workspace.numel()
                                                           * workspace.element_size())
+    # (named, so that a copy that contiguous() makes lives until the launch is queued)
+    q_scales, k_scales, v_scales = (q_scales.contiguous(), k_scales.contiguous(),
+                                    v_scales.contiguous())
     check(lib().reef_attention_prefill_int8(
-        C.byref(p), _ptr(q), C.byref(qs), _ptr(k), C.byref(ks), _ptr(v), C.byref(vs),
-        _ptr(q_scales.contiguous()), _ptr(k_scales.contiguous()), _ptr(v_scales.contiguous()),
-        _ptr(out), C.byref(os_), ws_ptr, ws_n, _stream()), "attention_prefill")
+        p, _ptr(q), qs, _ptr(k), ks, _ptr(v), vs, _ptr(q_scales), _ptr(k_scales), _ptr(v_scales),
+        _ptr(out), os_, ws_ptr, ws_n, stream), "attention_prefill")
     return out
 
 
@@ -355,28 +394,30 @@ def attention_prefill_cache(q, q_scales, k_cache, v_cache, k_scales, v_scales, k
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(D)
     start = kv_len - Sq if query_start is None else query_start
-    p = AttentionParams(B, Hq, Hkv, Sq, kv_len, D, start, window, softmax_scale, q_granularity,
-                        PER_TOKEN, 0)
+    p = _packed(_ATTENTION, AttentionParams, B, Hq, Hkv, Sq, kv_len, D, start, window,
+                softmax_scale, q_granularity, PER_TOKEN, 0)
     if block_table is None:
         max_context, table, max_blocks, pages = k_cache.shape[2], None, 0, 0
     else:
         max_context, table = 0, block_table.contiguous()
         max_blocks, pages = table.shape[1], k_cache.shape[0]
-    n = lib().reef_attention_prefill_cache_workspace_bytes(C.byref(p))
-    key = ("cache", torch.device(q.device).index, _stream().value)
+    n = lib().reef_attention_prefill_cache_workspace_bytes(p)
+    device, stream = q.device, _stream()
+    key = ("cache", device.index, stream)
     ws = _PREFILL_WS.get(key)
     if ws is None or ws.numel() < n:  # zero-filled once; every call leaves it so
-        ws = torch.zeros(max(n, 256), dtype=torch.uint8, device=q.device)
+        ws = torch.zeros(max(n, 256), dtype=torch.uint8, device=device)
         _PREFILL_WS[key] = ws
     if out is None:
         out = torch.empty((B, Hq, Sq, D), dtype=torch.float32, device=q.device)
     qs, os_ = _strides4(q), _strides4(out)
     own = status or StatusWord(q.device)
+    q_scales, k_cache, v_cache = q_scales.contiguous(), k_cache.contiguous(), v_cache.contiguous()
+    k_scales, v_scales = k_scales.contiguous(), v_scales.contiguous()
     check(lib().reef_attention_prefill_int8_cache(
-        C.byref(p), _ptr(q), C.byref(qs), _ptr(q_scales.contiguous()), _ptr(k_cache.contiguous()),
-        _ptr(v_cache.contiguous()), _ptr(k_scales.contiguous()), _ptr(v_scales.contiguous()),
-        max_context, _ptr(table), max_blocks, pages, _ptr(out), C.byref(os_), _ptr(ws), n,
-        own.ptr, _stream()), "attention_prefill_cache")
+        p, _ptr(q), qs, _ptr(q_scales), _ptr(k_cache), _ptr(v_cache), _ptr(k_scales),
+        _ptr(v_scales), max_context, _ptr(table), max_blocks, pages, _ptr(out), os_, _ptr(ws), n,
+        _ptr(own.tensor), stream), "attention_prefill_cache")
     if status is None:
         own.check("attention_prefill_cache")
     return out
@@ -419,6 +460,14 @@ def qk_scores_i32_packed(q, k):
     return acc
 
 
+def _decode_bytes(q, max_context, kv_heads, window, softmax_scale, q_granularity, num_splits):
+    B, Hq, D = q.shape
+    if softmax_scale is None:
+        softmax_scale = 1.0 / math.sqrt(D)
+    return _packed(_DECODE, DecodeParams, B, Hq, kv_heads, D, max_context, window, softmax_scale,
+                   q_granularity, num_splits, 0)
+
+
 def _decode_params(q, max_context, kv_heads, window, softmax_scale, q_granularity, num_splits):
     B, Hq, D = q.shape
     if softmax_scale is None:
@@ -430,8 +479,12 @@ def _decode_params(q, max_context, kv_heads, window, softmax_scale, q_granularit
 def decode_workspace(params: DecodeParams, device):
     """A zero-filled decode workspace (its item counters must start at zero; every
     launch leaves them so, so the workspace is reusable without refilling)."""
+    return _decode_workspace(C.byref(params), device)
+
+
+def _decode_workspace(params, device):
     torch = _torch()
-    n = lib().reef_attention_decode_workspace_bytes(C.byref(params))
+    n = lib().reef_attention_decode_workspace_bytes(params)
     return torch.zeros(max(n, 16) // 4 + 4, dtype=torch.float32, device=device)
 
 
@@ -449,16 +502,18 @@ def attention_decode(q, q_scales, k_cache, v_pages, k_scales, v_scales, context_
     Hkv, L = k_cache.shape[1], k_cache.shape[2]
     if tuple(k_cache.shape) != (B, Hkv, L, D) or v_pages.numel() != k_cache.numel():
         raise InvalidArgument("attention_decode cache shape mismatch")
-    p = _decode_params(q, L, Hkv, window, softmax_scale, q_granularity, num_splits)
-    ws = workspace if workspace is not None else decode_workspace(p, q.device)
+    p = _decode_bytes(q, L, Hkv, window, softmax_scale, q_granularity, num_splits)
+    ws = workspace if workspace is not None else _decode_workspace(p, q.device)
     if out is None:
         out = torch.empty((B, Hq, D), dtype=torch.float32, device=q.device)
     own = status or StatusWord(q.device)
     cl = context_lens.contiguous() if context_lens is not None else None
+    q, q_scales, k_cache, v_pages = (q.contiguous(), q_scales.contiguous(), k_cache.contiguous(),
+                                     v_pages.contiguous())
+    k_scales, v_scales = k_scales.contiguous(), v_scales.contiguous()
     check(lib().reef_attention_decode_int8(
-        C.byref(p), _ptr(q.contiguous()), _ptr(q_scales.contiguous()), _ptr(k_cache.contiguous()),
-        _ptr(v_pages.contiguous()), _ptr(k_scales.contiguous()), _ptr(v_scales.contiguous()),
-        _ptr(cl), _ptr(out), _ptr(ws), ws.numel() * 4, own.ptr, _stream()), "attention_decode")
+        p, _ptr(q), _ptr(q_scales), _ptr(k_cache), _ptr(v_pages), _ptr(k_scales), _ptr(v_scales),
+        _ptr(cl), _ptr(out), _ptr(ws), ws.numel() * 4, _ptr(own.tensor), _stream()), "attention_decode")
     if status is None:
         own.check("attention_decode")
     return out
@@ -476,17 +531,17 @@ def attention_decode_paged(q, q_scales, k_pages, v_pages, k_scale_pages, v_scale
     B, Hq, D = q.shape
     P, Hkv = k_pages.shape[0], k_pages.shape[1]
     max_blocks = block_table.shape[1]
-    p = _decode_params(q, max_blocks * PAGE, Hkv, window, softmax_scale, q_granularity,
-                       num_splits)
-    ws = workspace if workspace is not None else decode_workspace(p, q.device)
+    p = _decode_bytes(q, max_blocks * PAGE, Hkv, window, softmax_scale, q_granularity, num_splits)
+    ws = workspace if workspace is not None else _decode_workspace(p, q.device)
     if out is None:
         out = torch.empty((B, Hq, D), dtype=torch.float32, device=q.device)
     own = status or StatusWord(q.device)
+    q, q_scales, block_table, context_lens = (q.contiguous(), q_scales.contiguous(),
+                                              block_table.contiguous(), context_lens.contiguous())
     check(lib().reef_attention_decode_int8_paged(
-        C.byref(p), _ptr(q.contiguous()), _ptr(q_scales.contiguous()), _ptr(k_pages),
-        _ptr(v_pages), _ptr(k_scale_pages), _ptr(v_scale_pages), _ptr(block_table.contiguous()),
-        max_blocks, P, _ptr(context_lens.contiguous()), _ptr(out), _ptr(ws), ws.numel() * 4,
-        own.ptr, _stream()), "attention_decode_paged")
+        p, _ptr(q), _ptr(q_scales), _ptr(k_pages), _ptr(v_pages), _ptr(k_scale_pages),
+        _ptr(v_scale_pages), _ptr(block_table), max_blocks, P, _ptr(context_lens), _ptr(out),
+        _ptr(ws), ws.numel() * 4, _ptr(own.tensor), _stream()), "attention_decode_paged")
     if status is None:
         own.check("attention_decode_paged")
     return out
@@ -530,12 +585,12 @@ def kv_append(k_new, v_new, start_positions, k_cache, v_pages, k_scales, v_scale
     if tuple(k_cache.shape) != (B, H, L, D) or v_pages.numel() != k_cache.numel():
         raise InvalidArgument("KV cache append shape mismatch")
     _require(start_positions, torch.int32, "start_positions")
-    p = KvAppendParams(B, H, D, T, L)
+    p = _packed(_APPEND, KvAppendParams, B, H, D, T, L)
     own = status or StatusWord(k_new.device)
     check(lib().reef_kv_append_int8(
-        C.byref(p), _ptr(k_new), C.byref(ks), _ptr(v_new), C.byref(vs), _ptr(start_positions),
+        p, _ptr(k_new), ks, _ptr(v_new), vs, _ptr(start_positions),
         _ptr(k_cache), _ptr(v_pages), _ptr(k_scales), _ptr(v_scales), _ptr(context_lens),
-        own.ptr, _stream()), "kv_append")
+        _ptr(own.tensor), _stream()), "kv_append")
     if status is None:
         own.check("kv_append")
 
@@ -552,12 +607,12 @@ def kv_append_paged(k_new, v_new, start_positions, block_table, k_pages, v_pages
     max_blocks = block_table.shape[1]
     _require(start_positions, torch.int32, "start_positions")
     _require(block_table, torch.int32, "block_table")
-    p = KvAppendParams(B, H, D, T, max_context or max_blocks * PAGE)
+    p = _packed(_APPEND, KvAppendParams, B, H, D, T, max_context or max_blocks * PAGE)
+    block_table = block_table.contiguous()
     own = status or StatusWord(k_new.device)
     check(lib().reef_kv_append_int8_paged(
-        C.byref(p), _ptr(k_new), C.byref(ks), _ptr(v_new), C.byref(vs), _ptr(start_positions),
-        _ptr(block_table.contiguous()), max_blocks, P, _ptr(k_pages), _ptr(v_pages),
-        _ptr(k_scale_pages), _ptr(v_scale_pages), _ptr(context_lens), own.ptr, _stream()),
+        p, _ptr(k_new), ks, _ptr(v_new), vs, _ptr(start_positions), _ptr(block_table), max_blocks, P, _ptr(k_pages), _ptr(v_pages),
+        _ptr(k_scale_pages), _ptr(v_scale_pages), _ptr(context_lens), _ptr(own.tensor), _stream()),
         "kv_append_paged")
     if status is None:
         own.check("kv_append_paged")
@@ -578,13 +633,14 @@ def attention_int8_integer(q, k, v, table, *, score_shift, out_shift=8, query_st
     B, Hq, Sq, D = q.shape
     Hkv, Skv = k.shape[1], k.shape[2]
     start = Skv - Sq if query_start is None else query_start
-    p = AttentionParams(B, Hq, Hkv, Sq, Skv, D, start, window, 1.0, PER_HEAD, PER_HEAD, 0)
+    p = _packed(_ATTENTION, AttentionParams, B, Hq, Hkv, Sq, Skv, D, start, window, 1.0, PER_HEAD,
+                PER_HEAD, 0)
     out = torch.empty((B, Hq, Sq, D), dtype=torch.int8, device=q.device)
     sq, sk, sv, so = _strides4(q), _strides4(k), _strides4(v), _strides4(out)
+    table = table.contiguous()
     check(lib().reef_attention_int8_integer(
-        C.byref(p), _ptr(q), C.byref(sq), _ptr(k), C.byref(sk), _ptr(v), C.byref(sv),
-        score_shift, _ptr(table.contiguous()), out_shift, _ptr(out), C.byref(so), _stream()),
-        "attention_int8_integer")
+        p, _ptr(q), sq, _ptr(k), sk, _ptr(v), sv, score_shift, _ptr(table), out_shift, _ptr(out),
+        so, _stream()), "attention_int8_integer")
     return out
 
 
@@ -606,10 +662,11 @@ def linear_w8a8(x, weight, w_scales, bias=None, status: StatusWord | None = None
     ws = torch.empty(n // 4 + 4, dtype=torch.float32, device=x.device)
     y = torch.empty((rows, fout), dtype=torch.float32, device=x.device)
     own = status or StatusWord(x.device)
+    weight, w_scales = weight.contiguous(), w_scales.contiguous()
+    bias = bias.contiguous() if bias is not None else None
     check(lib().reef_linear_w8a8(
-        _ptr(x), rows, fin, x.stride(0), _ptr(weight.contiguous()), _ptr(w_scales.contiguous()),
-        _ptr(bias.contiguous()) if bias is not None else None, fout, _ptr(y), fout, _ptr(ws),
-        ws.numel() * 4, own.ptr, _stream()), "linear_w8a8")
+        _ptr(x), rows, fin, x.stride(0), _ptr(weight), _ptr(w_scales), _ptr(bias), fout, _ptr(y),
+        fout, _ptr(ws), ws.numel() * 4, _ptr(own.tensor), _stream()), "linear_w8a8")
     if status is None:
         own.check("linear_w8a8")
     return y
