@@ -159,11 +159,10 @@ reef_status reef_gemm_w8a8(const int8_t *xq, const float *x_scales, int64_t rows
  * workspace) returns REEF_INVALID_ARGUMENT, and PACKED outside the packed kernel's
  * limits REEF_UNSUPPORTED. AUTO takes PACKED for head_dim 128 with at least one
  * pair of 256-row query tiles per compute unit (and a workspace that holds the
- * image); of the others SPLIT for head_dim 128 and for grids of at most two 128-row
- * query tiles per compute unit, ONE_ITEM for larger grids at head_dim 64, and BALANCED,
- * with a large enough workspace, for at most one tile per compute unit whose heaviest
- * has many more keys than an equal share. AUTO takes SPLIT's kernel with PER_TOKEN K/V
- * scales too. Every schedule splits P into hi + lo where the values need it. */
+ * image); BALANCED with a large enough workspace and at most one 128-row query tile
+ * per compute unit; otherwise SPLIT for head_dim 128 and for small grids without a
+ * workspace, ONE_ITEM for head_dim 64 and with PER_TOKEN K/V scales. Every schedule
+ * splits P into hi + lo where the values need it. */
 #define REEF_ATTN_SCHED_MASK 0x70u
 #define REEF_ATTN_SCHED_AUTO 0x00u
 #define REEF_ATTN_SCHED_ONE_ITEM 0x10u /* one 128-row query tile per workgroup */
@@ -171,8 +170,8 @@ reef_status reef_gemm_w8a8(const int8_t *xq, const float *x_scales, int64_t rows
                                         * each tile's keys; hi + lo P */
 #define REEF_ATTN_SCHED_BALANCED 0x30u /* equal (tile, key block) ranges per workgroup,
                                         * two 4-wave groups splitting each range's key
-                                        * tiles; cut tiles merge through the workspace;
-                                        * hi + lo P */
+                                        * tiles (one with PER_TOKEN K/V scales); cut
+                                        * tiles merge through the workspace; hi + lo P */
 #define REEF_ATTN_SCHED_PACKED 0x40u   /* head_dim 128, per-tensor / per-head K and V
                                         * scales: V packed once into an fp16 image in the
                                         * workspace, 128-row query tiles, persistent

@@ -79,9 +79,7 @@ struct StreamPart {
     int64_t item_u0;  // first step of the item
 };
 
-template <int D> constexpr bool kFence = true;
-
-enum PrefillMode { kWhole, kSplit, kStream };
+enum PrefillMode { kWhole = 0, kSplit = 1, kStream = 2, kSplitStream = 3 };
 
 template <int D>
 struct StreamSlot {  // floats of one partial result: output in lane order, then (max, sum)
@@ -232,36 +230,31 @@ struct PrefillLds {
 };
 
 
-// MODE kWhole: one group of 4 waves computes all key tiles of the item. kSplit: the
-// workgroup is two groups of 4 waves over the same 128 query rows; group 0 takes the first
-// half of the key tiles and group 1 the second half, each with its own LDS stages, and
-// group 0 merges both partial results at the end. This halves the longest sequential
-// chain of a workgroup, which balances causal grids that fit the GPU at once, and gives
-// each SIMD two waves. kStream: the two groups split the key tiles [c0, c1) of one part of
-// an item, merge in LDS, and group 0 merges the parts of a cut item through the workspace
-// (StreamArgs) while group 1 joins its barriers. With one 4-wave group per part,
-// 4x32/8 chunk of 512 over 4096 keys, per-token scales: 336 us against 218.
+// SPLIT: the workgroup is two groups of 4 waves over the same 128 query rows;
+// group 0 takes the first half of the key tiles and group 1 the second half, each
+// with its own LDS stages, and group 0 merges both partial results at the end.
+// This halves the longest sequential chain of a workgroup, which balances causal
+// grids that fit the GPU at once.
+//
+// MODE kWhole and kStream compute key tiles [c0, c1) of the item (kWhole: all of
+// them); kStream parts of a cut item merge through the workspace (StreamArgs).
+// kSplitStream: the two groups of SPLIT split the key tiles [c0, c1) of a kStream
+// part, merge in LDS, and group 0 goes on as kStream (group 1 joins its barriers).
 template <int D, bool KV_TOKEN, int MODE>
 __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int b, int h, int c0,
                                              int c1, int8_t *smem_all,
-                                             float (*sScale_all)[KV_TOKEN ? 2 * kBN + 1 : 1],
+                                             float (*sScale)[KV_TOKEN ? 2 * kBN + 1 : 1],
                                              const StreamArgs &sa, const StreamPart &sp,
                                              uint32_t *sTicket) {
-    constexpr bool SPLIT = MODE != kWhole;
-    constexpr bool STREAM = MODE == kStream;
+    constexpr bool SPLIT = MODE == kSplit || MODE == kSplitStream;
+    constexpr bool STREAM = MODE == kStream || MODE == kSplitStream;
+    static_assert(!SPLIT || !KV_TOKEN, "the split kernels have no per-token K/V scales");
     constexpr int KSTRIDE = PrefillLds<D>::KSTRIDE, VSTRIDE = PrefillLds<D>::VSTRIDE;
     constexpr int DB = D / 32;  // 32-wide output blocks
     constexpr int K_BYTES = PrefillLds<D>::K_BYTES, V_BYTES = PrefillLds<D>::V_BYTES;
     constexpr int KLOADS = kBN * D / 16 / kThreads;  // 16-byte K loads per thread
     constexpr int VBLOCKS = (kBN / 4) * (D / 8);     // 4-key x 8-channel V blocks
-    // Rescale only when a row max grows by more than 2^kLazy. Per-token value scales vary
-    // the fp16 weights p s_v by themselves, so there p has less room to grow and the units
-    // more: p s_v kUnit / s_run stays below 2^15 (s_run within a factor 2 of the largest
-    // s_v), and since the matrix core takes subnormal fp16 parts as zero, a weight keeps
-    // its lo part down to 2^-13 of the row's largest (2^-9 with units of 2^6 and kLazy 8:
-    // 5.7e-6 relative error on 4x32/8 chunk of 512 over 4096 keys).
-    constexpr float kLazy = KV_TOKEN ? 4.0f : 8.0f;
-    constexpr float kUnit = 1024.0f;
+    constexpr float kLazy = 8.0f;  // rescale only when a row max grows by > 2^8
     // p = exp2(s - m_run + kShift): the row sums and the merges carry the same factor
     // 2^kShift, which cancels; it keeps a p of weight above 2^-21 of the row's
     // largest out of the fp16 subnormals (so hi and lo keep 11 bits each; below, each
@@ -275,7 +268,6 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int group = SPLIT ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
     int8_t *smem = smem_all + group * PrefillLds<D>::BYTES;
-    float(*sScale)[KV_TOKEN ? 2 * kBN + 1 : 1] = sScale_all + 2 * group;
     const int col = lane & 31, grp = lane >> 5;
     const int kvh = h / (a.q_heads / a.kv_heads);
     const int q0 = tile * kBM;
@@ -388,8 +380,8 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
     // This group's tiles: [kt0, kt0 + n_tiles * kBN); both groups run n_iter steps.
     int n_iter, kt0, n_tiles;
     if (SPLIT) {
-        const int s0 = STREAM ? c0 : 0;
-        const int n_seg = (STREAM ? min(c1, n_all) : n_all) - s0;
+        const int s0 = MODE == kSplitStream ? c0 : 0;
+        const int n_seg = (MODE == kSplitStream ? min(c1, n_all) : n_all) - s0;
         n_iter = (n_seg + 1) / 2;
         kt0 = kt_first + (s0 + (group ? n_iter : 0)) * kBN;
         n_tiles = group ? n_seg - n_iter : n_iter;
@@ -467,19 +459,19 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
                 grow = grow || svt > s_run * 2.0f;
             }
             // Lazy rescale: the running max only moves when some row's max grows by
-            // more than 2^kLazy (exp values stay <= 2^kLazy, well inside fp16).
+            // more than 2^kLazy (exp values stay <= 2^8, well inside fp16).
             if (__any(grow)) {
                 const float m_new = fmaxf(m_run, mt);
                 float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
                 float alpha_o = alpha;
                 if (KV_TOKEN) {
-                    // Values accumulate in units of s_run / kUnit, s_run the largest value
-                    // scale so far (within a factor 2), so that p * v_scale * kUnit / s_run
+                    // Values accumulate in units of s_run / 2^6, s_run the largest value
+                    // scale so far (within a factor 2), so that p * v_scale * 2^6 / s_run
                     // stays below 2^15 in fp16 and above its subnormals where its weight
                     // counts (the row sum is of p itself).
                     const float s_new = fmaxf(s_run, svt);
                     alpha_o = s_new > 0.0f ? alpha * (s_run / s_new) : alpha;
-                    inv_s = s_new > 0.0f ? kUnit / s_new : 0.0f;
+                    inv_s = s_new > 0.0f ? 64.0f / s_new : 0.0f;
                     s_run = s_new;
                 }
                 m_run = m_new;
@@ -603,15 +595,6 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
     for (; it < n_iter; ++it) step(it, std::false_type{});
 
     float l_tot = xor32_sum(l_run);
-    if (KV_TOKEN && SPLIT) {
-        // Groups and parts merge in absolute value units: the accumulator leaves the
-        // units of s_run (the largest value scale this group saw) here.
-#pragma unroll
-        for (int d = 0; d < DB; ++d)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[d][i] *= s_run * (1.0f / kUnit);
-        s_run = kUnit;
-    }
     if (SPLIT) {
         // Group 1 hands (running max, row sum, accumulator) to group 0 through LDS,
         // in a lane-linear layout (conflict-free 16-byte accesses).
@@ -629,7 +612,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
         __syncthreads();
         if (group == 1) {
             // the two barriers of group 0's part store and count below
-            if (STREAM && sp.parts > 1) {
+            if (MODE == kSplitStream && sp.parts > 1) {
                 __syncthreads();
                 __syncthreads();
             }
@@ -648,7 +631,16 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[d][4 * j + i] = acc[d][4 * j + i] * w0 + o[i] * w1;
             }
-        m_run = m;  // the merged state's maximum (a kStream part stores it)
+        m_run = m;  // the merged state's maximum (a kSplitStream part stores it)
+    }
+    if (KV_TOKEN && MODE == kStream) {
+        // Parts merge in absolute value units: the accumulator leaves the units of
+        // s_run (the largest value scale this part saw) here.
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[d][i] *= s_run * (1.0f / 64.0f);
+        s_run = 64.0f;
     }
     if (STREAM && sp.parts > 1) {
         // Leave this part in its slot (every lane: rows past q_len hold finite
@@ -740,7 +732,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
         l_tot = l;
     }
     if (!row_ok) return;
-    const float norm = (KV_TOKEN ? s_run * (1.0f / kUnit) : cv) / l_tot;
+    const float norm = (KV_TOKEN ? s_run * (1.0f / 64.0f) : cv) / l_tot;
     float *orow = a.out + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_st;
 #pragma unroll
     for (int d = 0; d < DB; ++d) {
@@ -759,12 +751,12 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
 // reverse order, so that with heaviest-first ranks every workgroup's sum of work
 // is about the same. A workgroup's next item starts while the stores of its last
 // one drain.
-template <int D, bool KV_TOKEN>
+template <int D>
 __global__ __launch_bounds__(2 * kThreads, 1) void prefill_split_kernel(PrefillArgs a, int items) {
     static_assert(4 * (D / 32) * 4 * kWave * 16 + 4 * kWave * 8 <= 2 * PrefillLds<D>::BYTES,
                   "merge buffer fits in the stages");
     __shared__ __attribute__((aligned(16))) int8_t smem[2 * PrefillLds<D>::BYTES];
-    __shared__ float sScale[4][KV_TOKEN ? 2 * kBN + 1 : 1];
+    __shared__ float sScale[2][1];
     const int G = gridDim.x;
     for (int r = 0;; ++r) {
         const int item = (r & 1) ? (r + 1) * G - 1 - (int)blockIdx.x : r * G + (int)blockIdx.x;
@@ -774,8 +766,8 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_split_kernel(PrefillA
         }
         int tile, b, h;
         item_coords(a, item, tile, b, h);
-        prefill_body<D, KV_TOKEN, kSplit>(a, tile, b, h, 0, 0, smem, sScale, StreamArgs{},
-                                          StreamPart{}, nullptr);
+        prefill_body<D, false, kSplit>(a, tile, b, h, 0, 0, smem, sScale, StreamArgs{},
+                                       StreamPart{}, nullptr);
         __syncthreads();  // the next item's stages overwrite the merge buffer
     }
 }
@@ -793,14 +785,18 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(PrefillArgs a) {
 // Balanced schedule (StreamArgs): workgroup g works through the steps
 // [L G^-1 units, (L + 1) G^-1 units) of logical workgroup L, where the G / 8
 // workgroups that run on one XCD (hardware workgroup g goes to XCD g % 8) hold
-// consecutive L, so an XCD's L2 sees a few heads, not all of them.
-template <int D, bool KV_TOKEN>
-__global__ __launch_bounds__(2 * kThreads, 1) void prefill_stream_kernel(PrefillArgs a,
-                                                                         StreamArgs sa) {
-    static_assert(4 * (D / 32) * 4 * kWave * 16 + 4 * kWave * 8 <= 2 * PrefillLds<D>::BYTES,
+// consecutive L, so an XCD's L2 sees a few heads, not all of them. GROUPS 2: the
+// workgroup is two 4-wave groups that split each part's key tiles (kSplitStream).
+template <int D, bool KV_TOKEN, int GROUPS>
+__global__ __launch_bounds__(GROUPS * kThreads, 1) void prefill_stream_kernel(
+    PrefillArgs a, StreamArgs sa) {
+    static_assert(GROUPS == 1 || (GROUPS == 2 && !KV_TOKEN), "two groups: no per-token scales");
+    static_assert(GROUPS == 1 || 4 * (D / 32) * 4 * kWave * 16 + 4 * kWave * 8 <=
+                                     2 * PrefillLds<D>::BYTES,
                   "merge buffer fits in the stages");
-    __shared__ __attribute__((aligned(16))) int8_t smem[2 * PrefillLds<D>::BYTES];
-    __shared__ float sScale[4][KV_TOKEN ? 2 * kBN + 1 : 1];
+    constexpr int MODE = GROUPS == 2 ? kSplitStream : kStream;
+    __shared__ __attribute__((aligned(16))) int8_t smem[GROUPS * PrefillLds<D>::BYTES];
+    __shared__ float sScale[2][KV_TOKEN ? 2 * kBN + 1 : 1];
     __shared__ uint32_t sTicket;
     const int G = gridDim.x, g = blockIdx.x;
     const int x = g % kXcds, per = G / kXcds, rem = G % kXcds;
@@ -834,7 +830,7 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_stream_kernel(Prefill
         sp.parts = wg_of(sp.item_u0 + n - 1) - sp.first_wg + 1;
         sp.slot = 2 * L + (first ? 0 : 1);
         sp.item = bh * a.q_tiles + tile;
-        prefill_body<D, KV_TOKEN, kStream>(a, tile, bh / a.q_heads, bh % a.q_heads, c0, c1, smem,
+        prefill_body<D, KV_TOKEN, MODE>(a, tile, bh / a.q_heads, bh % a.q_heads, c0, c1, smem,
                                         sScale, sa, sp, &sTicket);
         u += c1 - c0;
         c0 = 0;
@@ -923,7 +919,6 @@ constexpr int64_t kQueueWords = 16;  // the last words: the packed schedule's it
 constexpr int64_t kStreamMaxItems = kCounterWords - kQueueWords;
 constexpr int64_t kStreamMinSteps = 8;  // steps per workgroup of the balanced kernels
 constexpr int64_t kStreamCounterBytes = kCounterWords * 4;
-constexpr int64_t kBalanceSteps = 18;  // see the entry point's choice of a schedule
 
 int64_t stream_items(const reef_attention_params &p) {
     return ceil_div(p.q_len, kBM) * p.q_heads * p.batch;
@@ -1076,30 +1071,23 @@ extern "C" reef_status reef_attention_prefill_int8(
         return prefill_packed_launch(p, q, qst, k, kst, v, vst, q_scales, k_scales, v_scales, out,
                                      ost, static_cast<char *>(workspace) + bal_bytes, work, stream);
     }
-    // Among the other schedules the library takes
-    //   * balanced, which cuts the work of all items into equal ranges, for grids of at
-    //     most one 128-row tile per compute unit whose heaviest tile has kBalanceSteps key
-    //     tiles more than an equal range: that much longer the split kernel would run, at
-    //     1.2 us a key tile (1.6 with per-token scales, 0.8 at head_dim 64), and the cut
-    //     tiles' merges take about 20 us (1x8q/1kv x4096x128, 64 against 33: 61.4 against
-    //     80.3 us; 1x8x200x128, 4 against 8: 35 against 13.5 us);
-    //   * split, whose two 4-wave groups halve each tile's key loop, at head_dim 128
-    //     (1x32x2048x128: 60.5 us against 76.3 one-item; per-token scales, 4x32/8 chunk of
-    //     512 over 4096: 219 against 256, 2x32x2048x128: 154 against 165) and for small
-    //     grids at head_dim 64 (3x12x1021x64, window 256, per token: 22.0 against 27.6);
-    //   * one-item for larger grids at head_dim 64, where it holds two workgroups a unit
-    //     (4x16x2048x64: 67.8 us against 79.8; per token 102 against 117).
+    // The library takes the balanced schedule, which cuts the causal work of all
+    // items into equal ranges, for grids of at most one 128-row tile per compute unit
+    // (1x8q/1kv x4096x128: 63.6 us against 81.6 us with the split kernel and 92.5 us
+    // with the one-item kernel). On larger grids, head_dim 128 takes the split
+    // kernel, whose two 4-wave groups per workgroup halve each tile's key loop
+    // (1x32x2048x128: 65.9 us against 82.0 us one-item and 66.0 us balanced;
+    // 1x8q/1kv x8192x128: 195 against 278 us one-item),
+    // and head_dim 64 the one-item kernel (1x32x4096x64: 150 us against 160 us split,
+    // 4x32x4096x64: 541 against 582 us). Per-token K/V scales (which the split kernel
+    // does not take) use the one-item kernel; small grids without a workspace, the
+    // split kernel.
     if (sched == REEF_ATTN_SCHED_BALANCED && !stream_ok) return REEF_INVALID_ARGUMENT;
     if (sched == REEF_ATTN_SCHED_SPLIT && tok) return REEF_INVALID_ARGUMENT;
-    const int64_t per_head = host_steps_before(*p, a.q_tiles - 1) +
-                             host_tile_steps(*p, a.q_tiles - 1);
-    // The last whole tile sees the most keys (a partial one ends earlier).
-    const int64_t heaviest = std::max(host_tile_steps(*p, a.q_tiles - 1),
-                                      a.q_tiles > 1 ? host_tile_steps(*p, a.q_tiles - 2) : 0);
-    const int64_t range = std::max(kStreamMinSteps, per_head * p->batch * Hq / compute_units());
     if (sched == REEF_ATTN_SCHED_BALANCED ||
-        (sched == REEF_ATTN_SCHED_AUTO && stream_ok && items <= compute_units() &&
-         heaviest - range >= kBalanceSteps)) {
+        (sched == REEF_ATTN_SCHED_AUTO && stream_ok && items <= compute_units())) {
+        const int64_t per_head = host_steps_before(*p, a.q_tiles - 1) +
+                                 host_tile_steps(*p, a.q_tiles - 1);
         StreamArgs sa;
         sa.per_head = per_head;
         sa.units = per_head * p->batch * Hq;
@@ -1115,39 +1103,40 @@ extern "C" reef_status reef_attention_prefill_int8(
         const dim3 sgrid((unsigned)std::min<int64_t>(
             std::max<int64_t>(1, std::min<int64_t>(compute_units(), sa.units / kStreamMinSteps)),
             sa.units));
-#define REEF_STREAM_LAUNCH(DIM, TOK)                                                      \
-    hipLaunchKernelGGL((prefill_stream_kernel<DIM, TOK>), sgrid, dim3(2 * kThreads), 0, \
-                       stream, a, sa)
+        // Per-token K/V scales: one 4-wave group per workgroup; otherwise two groups
+        // that split each part's key tiles (two waves per SIMD).
         if (tok) {
-            if (D == 128) REEF_STREAM_LAUNCH(128, true);
-            else REEF_STREAM_LAUNCH(64, true);
+            if (D == 128)
+                hipLaunchKernelGGL((prefill_stream_kernel<128, true, 1>), sgrid, dim3(kThreads), 0,
+                                   stream, a, sa);
+            else
+                hipLaunchKernelGGL((prefill_stream_kernel<64, true, 1>), sgrid, dim3(kThreads), 0,
+                                   stream, a, sa);
         } else {
-            if (D == 128) REEF_STREAM_LAUNCH(128, false);
-            else REEF_STREAM_LAUNCH(64, false);
+            if (D == 128)
+                hipLaunchKernelGGL((prefill_stream_kernel<128, false, 2>), sgrid,
+                                   dim3(2 * kThreads), 0, stream, a, sa);
+            else
+                hipLaunchKernelGGL((prefill_stream_kernel<64, false, 2>), sgrid,
+                                   dim3(2 * kThreads), 0, stream, a, sa);
         }
-#undef REEF_STREAM_LAUNCH
         return launch_status();
     }
     const bool split = sched == REEF_ATTN_SCHED_SPLIT ||
-                       (sched == REEF_ATTN_SCHED_AUTO &&
-                        (D == 128 || items <= 2 * compute_units()));
+                       (sched == REEF_ATTN_SCHED_AUTO && !tok &&
+                        (items <= compute_units() || D == 128));
     // The 4-wave kernel places two workgroups on each of the 256 compute units at
     // once; zig-zag pairs a heavy and a light tile there. The split kernel holds a
     // compute unit alone and takes the tiles heaviest first.
     a.zigzag = !split && items <= 2 * compute_units() ? 1 : 0;
     if (split) {
         const dim3 pgrid((unsigned)std::min<int64_t>(items, compute_units()));
-#define REEF_SPLIT_LAUNCH(DIM, TOK)                                                             \
-    hipLaunchKernelGGL((prefill_split_kernel<DIM, TOK>), pgrid, dim3(2 * kThreads), 0, stream, a, \
-                       (int)items)
-        if (tok) {
-            if (D == 128) REEF_SPLIT_LAUNCH(128, true);
-            else REEF_SPLIT_LAUNCH(64, true);
-        } else {
-            if (D == 128) REEF_SPLIT_LAUNCH(128, false);
-            else REEF_SPLIT_LAUNCH(64, false);
-        }
-#undef REEF_SPLIT_LAUNCH
+        if (D == 128)
+            hipLaunchKernelGGL(prefill_split_kernel<128>, pgrid, dim3(2 * kThreads), 0, stream, a,
+                               (int)items);
+        else
+            hipLaunchKernelGGL(prefill_split_kernel<64>, pgrid, dim3(2 * kThreads), 0, stream, a,
+                               (int)items);
         return launch_status();
     }
 #define REEF_PREFILL_LAUNCH(DIM, TOK) \
