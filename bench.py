@@ -199,16 +199,21 @@ def prefill_kernels(torch, cfg):
     or per-head scales, a workspace): the packed schedule (a V-image pack, then the
     attention kernel) when head_dim is 128 and there is at least one pair of 256-row
     query tiles per compute unit; the balanced schedule with at most one 128-row
-    query tile per compute unit; otherwise the split kernel at head_dim 128 and the
-    one-item kernel at 64. Each is one launch; the packed kernel splits P into fp16
+    query tile per compute unit whose heaviest has 18 key tiles more than an equal share;
+    otherwise the split kernel at head_dim 128 and on such small grids, the one-item
+    kernel at 64. Each is one launch; the packed kernel splits P into fp16
     hi + lo parts for the heads whose values need it, the others always."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     pairs = ((cfg.seq + 255) // 256 + 1) // 2 * cfg.batch * cfg.q_heads
     if cfg.head_dim == 128 and pairs >= cus:
         return "vt_pack_kernel + prefill_packed_kernel"
-    if (cfg.seq + 127) // 128 * cfg.batch * cfg.q_heads <= cus:
+    tiles = (cfg.seq + 127) // 128
+    items = tiles * cfg.batch * cfg.q_heads
+    steps = [(min(128 * (t + 1), cfg.seq) + 63) // 64 for t in range(tiles)]
+    share = max(8, sum(steps) * cfg.batch * cfg.q_heads // cus)
+    if items <= cus and max(steps) - share >= 18:
         return "prefill_stream_kernel"
-    return "prefill_split_kernel" if cfg.head_dim == 128 else "prefill_kernel"
+    return "prefill_split_kernel" if cfg.head_dim == 128 or items <= cus else "prefill_kernel"
 
 
 def bench_prefill(torch, reef, W, name, steps, warmup, with_quant=True):

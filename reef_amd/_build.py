@@ -30,10 +30,12 @@ FLAGS = [
 ]
 
 
-# Per source: matrix products with their accumulators in ordinary vector registers. The
-# GEMM's smaller tiles need no others; left to itself the compiler moves accumulators
-# between the two register files on every K step (120 moves beside 40 products).
-SOURCE_FLAGS = {"linear.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# Per source: matrix products with their accumulators in ordinary vector registers. Left to
+# itself the compiler moves accumulators between the two register files inside the loops:
+# 120 moves beside 40 products of the GEMM's smaller tiles, and the one-item prefill takes
+# 4 to 7 % longer at head_dim 64 (1x32x2048x64: 47.4 us against 44.2).
+VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+SOURCE_FLAGS = {"linear.hip": VGPR_FORM, "prefill.hip": VGPR_FORM}
 
 
 def commands(objdir):

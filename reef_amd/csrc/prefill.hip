@@ -772,8 +772,13 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_split_kernel(PrefillA
     }
 }
 
+// Two workgroups share a compute unit, so each SIMD has two waves to fill each other's
+// waits; at head_dim 128 that holds a wave to 256 registers (43 spilled outside the key
+// loop's steady state with per-token scales, 12 without), against 285 and one wave: 4x32/8
+// chunk of 512 over 4096 keys, per token, 207 us against 262; 2x32x2048x128 129 against
+// 167; 1x32x2048x128 per head 61 against 76.
 template <int D, bool KV_TOKEN>
-__global__ __launch_bounds__(kThreads, 1) void prefill_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(kThreads, 2) void prefill_kernel(PrefillArgs a) {
     __shared__ __attribute__((aligned(16))) int8_t smem[PrefillLds<D>::BYTES];
     __shared__ float sScale[2][KV_TOKEN ? 2 * kBN + 1 : 1];
     int tile, b, h;
@@ -919,6 +924,7 @@ constexpr int64_t kQueueWords = 16;  // the last words: the packed schedule's it
 constexpr int64_t kStreamMaxItems = kCounterWords - kQueueWords;
 constexpr int64_t kStreamMinSteps = 8;  // steps per workgroup of the balanced kernels
 constexpr int64_t kStreamCounterBytes = kCounterWords * 4;
+constexpr int64_t kBalanceSteps = 18;  // see the entry point's choice of a schedule
 
 int64_t stream_items(const reef_attention_params &p) {
     return ceil_div(p.q_len, kBM) * p.q_heads * p.batch;
@@ -1071,23 +1077,31 @@ extern "C" reef_status reef_attention_prefill_int8(
         return prefill_packed_launch(p, q, qst, k, kst, v, vst, q_scales, k_scales, v_scales, out,
                                      ost, static_cast<char *>(workspace) + bal_bytes, work, stream);
     }
-    // The library takes the balanced schedule, which cuts the causal work of all
-    // items into equal ranges, for grids of at most one 128-row tile per compute unit
-    // (1x8q/1kv x4096x128: 63.6 us against 81.6 us with the split kernel and 92.5 us
-    // with the one-item kernel). On larger grids, head_dim 128 takes the split
-    // kernel, whose two 4-wave groups per workgroup halve each tile's key loop
-    // (1x32x2048x128: 65.9 us against 82.0 us one-item and 66.0 us balanced;
-    // 1x8q/1kv x8192x128: 195 against 278 us one-item),
-    // and head_dim 64 the one-item kernel (1x32x4096x64: 150 us against 160 us split,
-    // 4x32x4096x64: 541 against 582 us). Per-token K/V scales (which the split kernel
-    // does not take) use the one-item kernel; small grids without a workspace, the
-    // split kernel.
+    // Among the other schedules the library takes
+    //   * balanced, which cuts the work of all items into equal ranges, for grids of at
+    //     most one 128-row tile per compute unit whose heaviest tile has kBalanceSteps key
+    //     tiles more than an equal range: that much longer the split kernel would run, at
+    //     1.2 us a key tile (0.8 at head_dim 64), and the cut tiles' merges take about 20 us
+    //     (1x8q/1kv x4096x128, 64 against 33: 61.4 us against 80.3; 1x8x2048x128, 32 against
+    //     8: 35 against 45; 1x8x1024x128, 16 against 8: 31.5 against 27.9; 1x8x200x128, 4
+    //     against 8: 35 against 13.5);
+    //   * split, whose two 4-wave groups halve each tile's key loop, for smaller grids and
+    //     at head_dim 128 (1x32x2048x128: 60.5 us against 76.3 one-item; 1x8q/1kv x8192x128:
+    //     195 against 278);
+    //   * one-item for larger grids at head_dim 64, where it holds two workgroups a unit
+    //     (1x32x2048x64: 45.8 us against 46.5 split; 4x16x2048x64: 67.8 against 79.8).
+    // Per-token K/V scales take balanced for at most one tile per unit, one-item otherwise.
     if (sched == REEF_ATTN_SCHED_BALANCED && !stream_ok) return REEF_INVALID_ARGUMENT;
     if (sched == REEF_ATTN_SCHED_SPLIT && tok) return REEF_INVALID_ARGUMENT;
+    const int64_t per_head = host_steps_before(*p, a.q_tiles - 1) +
+                             host_tile_steps(*p, a.q_tiles - 1);
+    // The last whole tile sees the most keys (a partial one ends earlier).
+    const int64_t heaviest = std::max(host_tile_steps(*p, a.q_tiles - 1),
+                                      a.q_tiles > 1 ? host_tile_steps(*p, a.q_tiles - 2) : 0);
+    const int64_t range = std::max(kStreamMinSteps, per_head * p->batch * Hq / compute_units());
     if (sched == REEF_ATTN_SCHED_BALANCED ||
-        (sched == REEF_ATTN_SCHED_AUTO && stream_ok && items <= compute_units())) {
-        const int64_t per_head = host_steps_before(*p, a.q_tiles - 1) +
-                                 host_tile_steps(*p, a.q_tiles - 1);
+        (sched == REEF_ATTN_SCHED_AUTO && stream_ok && items <= compute_units() &&
+         (tok || heaviest - range >= kBalanceSteps))) {
         StreamArgs sa;
         sa.per_head = per_head;
         sa.units = per_head * p->batch * Hq;

@@ -388,6 +388,24 @@ def test_prefill_matches_oracle(reef, B, Hq, Hkv, Sq, Skv, D, start, window, gq,
         assert err <= TOL, (precise, sched, ws, err)
 
 
+@pytest.mark.parametrize("S", [1600, 1664])
+@pytest.mark.parametrize("D,start", [(64, 0), (128, 0), (128, 130)])
+def test_prefill_schedule_threshold(reef, S, D, start):
+    """Grids of at most one tile per compute unit on both sides of the library's line
+    between the split and the balanced schedule (the heaviest of 13 tiles has 25 and 26
+    key tiles against an equal range of 8; with 130 keys before the first row, 27 and 28)."""
+    case(f"prefill schedule threshold S{S} D{D} start{start}")
+    B, H = 1, 1
+    q = W.lcg_normal(811 + S, B * H * S * D).reshape(B, H, S, D)
+    k = W.lcg_normal(812 + S, B * H * (S + start) * D).reshape(B, H, S + start, D)
+    v = W.lcg_normal(813 + S, B * H * (S + start) * D).reshape(B, H, S + start, D)
+    p = oracle.Problem(B, H, H, S, S + start, D, softmax_scale=1 / math.sqrt(D))
+    out, gold = _run_prefill(reef, q, k, v, p)
+    err = np.abs(out - gold).max()
+    print(f"max_abs_err {err:.3e}", flush=True)
+    assert err <= 1e-5  # hi + lo P: 22 bits of weights whose values reach about 4
+
+
 def test_prefill_outlier_channels(reef):
     """Per-head scales with a few value channels scaled x8 (activation outliers):
     the values of those heads reach |v| ~ 30, where one fp16 P is not precise enough.
