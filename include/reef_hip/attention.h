@@ -98,6 +98,16 @@ reef_status reef_quantize_int8_per_token(const float *x, int64_t rows, int64_t w
                                          int64_t row_stride, int8_t *q, float *scales,
                                          uint32_t *status_word, hipStream_t stream);
 
+/* The same rows out of a strided [B, H, S, D] tensor (NULL: packed), in [B, H, S]
+ * order: q packed [B, H, S, D], scales [B, H, S]. Whole 16-byte rows only (head_dim and
+ * strides multiples of 4, x on 16 bytes, head_dim at most 1024): REEF_UNSUPPORTED
+ * otherwise. */
+reef_status reef_quantize_int8_per_token_heads(const float *x, int64_t batch, int64_t heads,
+                                               int64_t tokens, int64_t head_dim,
+                                               const reef_strides *x_strides, int8_t *q,
+                                               float *scales, uint32_t *status_word,
+                                               hipStream_t stream);
+
 /* Dequantize: x[i] = float(q[i]) * scale[i / group] (group = width for
  * per-token rows, n for per-tensor). */
 reef_status reef_dequantize_int8(const int8_t *q, int64_t n, int64_t group, const float *scales,

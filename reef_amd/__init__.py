@@ -32,7 +32,8 @@ PAGE = 16
 
 EXPORTS = [
     "reef_quantize_int8_per_tensor", "reef_quantize_int8_per_head",
-    "reef_quantize_int8_per_token", "reef_dequantize_int8", "reef_read_status_word",
+    "reef_quantize_int8_per_token", "reef_quantize_int8_per_token_heads",
+    "reef_dequantize_int8", "reef_read_status_word",
     "reef_attention_prefill_workspace_bytes", "reef_attention_prefill_int8", "reef_qk_scores_i32",
     "reef_qk_scores_i32_packed_workspace_bytes", "reef_qk_scores_i32_packed",
     "reef_attention_decode_workspace_bytes", "reef_attention_decode_int8",
@@ -108,6 +109,7 @@ _SIGS = {
     "reef_quantize_int8_per_tensor": [_P, _I64, _P, _P, _P, _P],
     "reef_quantize_int8_per_head": [_P, _I64, _I64, _I64, _I64, _S, _P, _P, _P, _P],
     "reef_quantize_int8_per_token": [_P, _I64, _I64, _I64, _P, _P, _P, _P],
+    "reef_quantize_int8_per_token_heads": [_P, _I64, _I64, _I64, _I64, _S, _P, _P, _P, _P],
     "reef_dequantize_int8": [_P, _I64, _I64, _P, _P, _P],
     "reef_read_status_word": [_P, C.c_int, _P],
     "reef_attention_prefill_workspace_bytes": [_S],
@@ -280,6 +282,19 @@ def quantize_rows(x, status: StatusWord | None = None):
     _require(x, torch.float32, "x")
     shape = x.shape
     width = shape[-1]
+    if len(shape) == 4 and not x.is_contiguous() and x.numel() > 0:
+        # heads as a projection lays them out: read in place rather than copied first
+        sb, sh, st, sd = x.stride()
+        if sd == 1 and (sb | sh | st | width) % 4 == 0 and width <= 1024 and x.data_ptr() % 16 == 0:
+            q = torch.empty(shape, dtype=torch.int8, device=x.device)
+            s = torch.empty(shape[:-1], dtype=torch.float32, device=x.device)
+            own = status or StatusWord(x.device)
+            check(lib().reef_quantize_int8_per_token_heads(
+                _ptr(x), *shape, _STRIDES.pack(sb, sh, st), _ptr(q), _ptr(s), _ptr(own.tensor),
+                _stream()), "quantize_rows")
+            if status is None:
+                own.check("quantize_rows requires finite values")
+            return q, s
     x2 = x if len(shape) == 2 else x.reshape(-1, width)
     if x2.stride(1) != 1:
         x2 = x2.contiguous()

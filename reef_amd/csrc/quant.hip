@@ -470,9 +470,18 @@ __host__ __device__ constexpr int row_groups(int per, bool nt) {
     return nt && per < 4 ? 4 / per : 1;
 }
 
-template <int LPR, int PER, bool NT>
+// Rows are row_stride apart or, kHeads, the [batch, heads, tokens] rows of a strided
+// tensor (HeadRows): a row's place costs two divisions, and the rows need no copy into
+// order first (4x32x512x128 queries from a projection's [B, S, H, D]: a copy of 12.6 us
+// and 9.9 us before, 12.6 us in all now).
+struct HeadRows {
+    int64_t sb, sh, st;  // element strides of batch, head, token
+    int32_t heads, tokens;
+};
+
+template <int LPR, int PER, bool NT, bool kHeads>
 __global__ __launch_bounds__(kQuantThreads) void token_quantize_regs(
-    const float *__restrict__ x, int64_t rows, int32_t w4, int64_t row_stride,
+    const float *__restrict__ x, int64_t rows, int32_t w4, int64_t row_stride, HeadRows hr,
     int8_t *__restrict__ q, float *__restrict__ scales, uint32_t *status) {
     constexpr int RPW = kWave / LPR;  // rows per wave and group
     constexpr int G = row_groups(PER, NT);
@@ -483,7 +492,13 @@ __global__ __launch_bounds__(kQuantThreads) void token_quantize_regs(
     for (int g = 0; g < G; ++g) {
         const int64_t row = (wave_id * G + g) * RPW + sub;
         const bool live = row < rows;
-        const float4 *r = reinterpret_cast<const float4 *>(x + (live ? row : 0) * row_stride);
+        int64_t off = (live ? row : 0) * row_stride;
+        if constexpr (kHeads) {
+            const uint32_t n = live ? (uint32_t)row : 0u, bh = n / (uint32_t)hr.tokens,
+                           b = bh / (uint32_t)hr.heads;
+            off = b * hr.sb + (bh - b * hr.heads) * hr.sh + (n - bh * hr.tokens) * hr.st;
+        }
+        const float4 *r = reinterpret_cast<const float4 *>(x + off);
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
             const int col = l + j * LPR;
@@ -688,10 +703,10 @@ void launch_block(const FlatHeads &f, int8_t *q, float *scales, uint32_t *status
 }
 
 // The register and wide forms (width % 4 == 0, w4 = width / 4 <= 8 * kQuantThreads).
-template <bool NT>
-void launch_rows(const float *x, int64_t rows, int64_t w4, int64_t row_stride, int8_t *q,
-                 float *scales, uint32_t *status_word, hipStream_t stream) {
-    if (w4 <= 4 * kWave) {
+template <bool NT, bool kHeads>
+void launch_rows(const float *x, int64_t rows, int64_t w4, int64_t row_stride, const HeadRows &hr,
+                 int8_t *q, float *scales, uint32_t *status_word, hipStream_t stream) {
+    if (kHeads || w4 <= 4 * kWave) {
         // lanes per row: the smallest power of two >= w4 (up to 64), then up to 4
         // float4 per lane
         int lpr = 1;
@@ -701,8 +716,8 @@ void launch_rows(const float *x, int64_t rows, int64_t w4, int64_t row_stride, i
             (int64_t)(kWave / lpr) * row_groups(per, NT) * (kQuantThreads / kWave);
         const dim3 grid((unsigned)ceil_div(rows, rows_per_block));
 #define REEF_TOKEN_LAUNCH(L, P)                                                               \
-    hipLaunchKernelGGL((token_quantize_regs<L, P, NT>), grid, dim3(kQuantThreads), 0, stream, \
-                       x, rows, (int32_t)w4, row_stride, q, scales, status_word)
+    hipLaunchKernelGGL((token_quantize_regs<L, P, NT, kHeads>), grid, dim3(kQuantThreads), 0, \
+                       stream, x, rows, (int32_t)w4, row_stride, hr, q, scales, status_word)
         switch (lpr) {
         case 1: REEF_TOKEN_LAUNCH(1, 1); break;
         case 2: REEF_TOKEN_LAUNCH(2, 1); break;
@@ -866,14 +881,44 @@ extern "C" reef_status reef_quantize_int8_per_token(const float *x, int64_t rows
     const int64_t w4 = width / 4;
     if (vec && (w4 <= 4 * kWave || (w4 <= 8 * kQuantThreads && rows < (int64_t(1) << 31)))) {
         if (4 * rows * row_stride > kStreamBytes)
-            launch_rows<true>(x, rows, w4, row_stride, q, scales, status_word, stream);
+            launch_rows<true, false>(x, rows, w4, row_stride, HeadRows{}, q, scales, status_word,
+                                     stream);
         else
-            launch_rows<false>(x, rows, w4, row_stride, q, scales, status_word, stream);
+            launch_rows<false, false>(x, rows, w4, row_stride, HeadRows{}, q, scales, status_word,
+                                      stream);
     } else {
         const dim3 grid((unsigned)ceil_div(rows, kQuantThreads / kWave));
         hipLaunchKernelGGL(token_quantize, grid, dim3(kQuantThreads), 0, stream, x, rows, width,
                            row_stride, q, scales, status_word);
     }
+    return launch_status();
+}
+
+extern "C" reef_status reef_quantize_int8_per_token_heads(const float *x, int64_t batch,
+                                                          int64_t heads, int64_t tokens,
+                                                          int64_t head_dim,
+                                                          const reef_strides *xs, int8_t *q,
+                                                          float *scales, uint32_t *status_word,
+                                                          hipStream_t stream) {
+    if (!x || !q || !scales || batch <= 0 || heads <= 0 || tokens <= 0 || head_dim <= 0)
+        return REEF_INVALID_ARGUMENT;
+    HeadRows hr;
+    hr.sb = xs ? xs->batch : heads * tokens * head_dim;
+    hr.sh = xs ? xs->head : tokens * head_dim;
+    hr.st = xs ? xs->token : head_dim;
+    if (hr.sb < 0 || hr.sh < 0 || hr.st < 0) return REEF_INVALID_ARGUMENT;
+    // whole float4 rows held in a wave's registers, rows counted in 31 bits
+    if (head_dim % 4 != 0 || head_dim > 16 * kWave || hr.sb % 4 != 0 || hr.sh % 4 != 0 ||
+        hr.st % 4 != 0 || !aligned(x, 16) || !aligned(q, 4) ||
+        heads >= (int64_t(1) << 31) / tokens || batch >= (int64_t(1) << 31) / (heads * tokens))
+        return REEF_UNSUPPORTED;
+    hr.heads = (int32_t)heads;
+    hr.tokens = (int32_t)tokens;
+    const int64_t rows = batch * heads * tokens;
+    if (4 * rows * head_dim > kStreamBytes)
+        launch_rows<true, true>(x, rows, head_dim / 4, 0, hr, q, scales, status_word, stream);
+    else
+        launch_rows<false, true>(x, rows, head_dim / 4, 0, hr, q, scales, status_word, stream);
     return launch_status();
 }
 

@@ -212,6 +212,31 @@ def test_quantize_rows_with_row_stride(reef):
     assert np.array_equal(host(q), qo) and np.array_equal(host(s), so)
 
 
+@pytest.mark.parametrize("B,H,S,D", [(2, 3, 37, 128), (1, 12, 5, 64), (3, 2, 1, 4), (1, 2, 9, 1024),
+                                     (2, 2, 7, 36), (2, 3, 7, 1028), (2, 3, 7, 6)])
+def test_quantize_rows_of_strided_heads_bit_exact(reef, B, H, S, D):
+    """The heads of a projection [B, S, H, D] read in place (every lane and register
+    count of the row kernel), and the widths that are copied into order first (wider than
+    1024 or not in whole float4): codes, scales and layout as of the copied tensor; an
+    expanded tensor (stride 0) too."""
+    case(f"quantize_rows of strided heads [{B}, {H}, {S}, {D}]")
+    x = W.lcg_normal(31 + D, B * S * H * D).reshape(B, S, H, D)
+    x *= W.lcg_uniform(32, B * S * H, 0.01, 40.0).reshape(B, S, H, 1)
+    xt = gpu(x).permute(0, 2, 1, 3)
+    q, s = reef.quantize_rows(xt)
+    qo, so = oracle.quantize_rows(np.ascontiguousarray(x.transpose(0, 2, 1, 3)).reshape(-1, D))
+    assert q.is_contiguous() and s.is_contiguous()
+    assert np.array_equal(host(q).reshape(-1, D), qo)
+    assert np.array_equal(host(s).reshape(-1).view(np.uint32), so.view(np.uint32))
+    e = gpu(x)[:, :1].expand(B, S, H, D).permute(0, 2, 1, 3)
+    q, s = reef.quantize_rows(e)
+    qo, so = oracle.quantize_rows(host(e).reshape(-1, D))
+    assert np.array_equal(host(q).reshape(-1, D), qo)
+    x[B - 1, S - 1, H - 1, D - 1] = np.nan
+    with pytest.raises(ValueError):
+        reef.quantize_rows(gpu(x).permute(0, 2, 1, 3))
+
+
 @pytest.mark.parametrize("n,group", [(4096 * 128, 128), (1_000_003, 1_000_003), (77, 7),
                                      (3 * 8193, 8193), (4 * 61, 61), (1, 1), (10, 4)])
 def test_dequantize_bit_exact(reef, n, group):
