@@ -35,7 +35,7 @@ FLAGS = [
 # 120 moves beside 40 products of the GEMM's smaller tiles, and the one-item prefill takes
 # 4 to 7 % longer at head_dim 64 (1x32x2048x64: 47.4 us against 44.2).
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-SOURCE_FLAGS = {"linear.hip": VGPR_FORM, "prefill.hip": VGPR_FORM}
+SOURCE_FLAGS = {"linear.hip": VGPR_FORM, "prefill.hip": VGPR_FORM, "int_head.hip": VGPR_FORM}
 
 
 def commands(objdir):

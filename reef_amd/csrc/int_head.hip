@@ -77,18 +77,29 @@ struct IntLds {
     static constexpr int K_PER_THREAD = (K_CHUNKS + kIntThreads - 1) / kIntThreads;
 };
 
-template <int D>
-__global__ __launch_bounds__(kIntThreads, 2) void int_head_kernel(IntHeadArgs a) {
+// A workgroup is G groups of 4 waves over the same 128 query rows; group g takes key tiles
+// g, g + G, ... with LDS tiles of its own. Maxima, weight sums and products are integers,
+// so the groups' results merge exactly through LDS, in any order. The three walks over
+// the keys are one serial chain per tile, which groups shorten (see the launch).
+template <int D, int G>
+__global__ __launch_bounds__(G * kIntThreads, 1) void int_head_kernel(IntHeadArgs a) {
     using L = IntLds<D>;
     constexpr int DB = D / 32;
+    struct Tiles {
+        int8_t k[2][L::K_BYTES];
+        _Float16 v[2][D * L::V_ROW];
+    };
     __shared__ uint16_t sTable[256];
-    __shared__ __attribute__((aligned(16))) int8_t sK[2][L::K_BYTES];
-    __shared__ __attribute__((aligned(16))) _Float16 sV[2][D * L::V_ROW];
+    __shared__ uint32_t sRow[G][kIntRows];
+    __shared__ __attribute__((aligned(16))) Tiles sTiles[G];
 
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x & (kIntThreads - 1), lane = tid & 63;
+    const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kIntThreads);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, grp = lane >> 5;
-    sTable[tid] = a.table[tid];  // 256 threads, 256 entries
+    auto &sK = sTiles[group].k;
+    auto &sV = sTiles[group].v;
+    if (threadIdx.x < 256) sTable[threadIdx.x] = a.table[threadIdx.x];
 
     const int pairs = a.batch * a.q_heads;
     const int tile = a.q_tiles - 1 - (int)blockIdx.x / pairs;  // heaviest first
@@ -173,15 +184,21 @@ __global__ __launch_bounds__(kIntThreads, 2) void int_head_kernel(IntHeadArgs a)
     // loads in flight meanwhile), then f(kt, buf) runs for the wave's own tiles.
     // extra_load(kt) / extra_store(buf) stage more per-tile data the same way.
     auto walk = [&](auto f, auto extra_load, auto extra_store) {
-        load_k(kt0);
-        extra_load(kt0);
-        int buf = 0;
-        for (int kt = kt0; kt <= key_hi; kt += kIntKeys, buf ^= 1) {
-            store_k(buf);
-            extra_store(buf);
-            if (kt + kIntKeys <= key_hi) {
-                load_k(kt + kIntKeys);
-                extra_load(kt + kIntKeys);
+        constexpr int kStep = G * kIntKeys;
+        int kt = kt0 + group * kIntKeys, buf = 0;
+        if (kt <= key_hi) {
+            load_k(kt);
+            extra_load(kt);
+        }
+        // every group runs the same number of barriers
+        for (int first = kt0; first <= key_hi; first += kStep, kt += kStep, buf ^= 1) {
+            if (kt <= key_hi) {
+                store_k(buf);
+                extra_store(buf);
+            }
+            if (kt + kStep <= key_hi) {
+                load_k(kt + kStep);
+                extra_load(kt + kStep);
             }
             // the stores are visible; every wave has finished reading this buffer's
             // previous tile (it did so before the last barrier)
@@ -189,6 +206,18 @@ __global__ __launch_bounds__(kIntThreads, 2) void int_head_kernel(IntHeadArgs a)
             if (kt >= wt0 && kt <= wt1) f(kt, buf);
         }
         __syncthreads();  // the next walk's first stores reuse the buffers
+    };
+    // The groups' values of this lane's row, in every group (f folds two of them).
+    auto over_groups = [&](uint32_t value, auto f) {
+        if constexpr (G > 1) {
+            if (grp == 0) sRow[group][32 * wave + col] = value;
+            __syncthreads();
+            value = sRow[0][32 * wave + col];
+#pragma unroll
+            for (int g = 1; g < G; ++g) value = f(value, sRow[g][32 * wave + col]);
+            __syncthreads();  // sRow is written again
+        }
+        return value;
     };
     auto no_load = [](int) {};
     auto no_store = [](int) {};
@@ -216,6 +245,9 @@ __global__ __launch_bounds__(kIntThreads, 2) void int_head_kernel(IntHeadArgs a)
         const auto sw = __builtin_amdgcn_permlane32_swap((uint32_t)mx, (uint32_t)mx, false, false);
         mx = max((int32_t)sw[0], (int32_t)sw[1]);
     }
+    mx = (int32_t)over_groups((uint32_t)mx, [](uint32_t x, uint32_t y) {
+        return (uint32_t)max((int32_t)x, (int32_t)y);
+    });
 
     // Pass 2: the sum of table weights (:208-217).
     uint32_t sum = 0;
@@ -244,6 +276,7 @@ __global__ __launch_bounds__(kIntThreads, 2) void int_head_kernel(IntHeadArgs a)
         const auto sw = __builtin_amdgcn_permlane32_swap(sum, sum, false, false);
         sum = sw[0] + sw[1];
     }
+    sum = over_groups(sum, [](uint32_t x, uint32_t y) { return x + y; });
     // The maximum's weight is the table's first entry, so sum > 0 on a row that
     // sees a key; rows outside the tensor never store.
     const uint32_t recip = sum > 0 ? (255u << 16) / sum : 0u;
@@ -328,6 +361,34 @@ __global__ __launch_bounds__(kIntThreads, 2) void int_head_kernel(IntHeadArgs a)
             }
     }, load_v, store_v);
 
+    if constexpr (G > 1) {
+        // Groups 1 .. G - 1 leave their products in LDS, lane-linear (conflict-free 16-byte
+        // accesses) over all of the tiles, which the walk's last barrier has freed; group 0
+        // adds them, integers below 2^24 like their sum.
+        constexpr int kPart = 4 * DB * 4 * 64;  // f32x4 per group
+        static_assert((G - 1) * kPart * sizeof(f32x4) <= sizeof(sTiles), "products fit the tiles");
+        f32x4 *parts = reinterpret_cast<f32x4 *>(&sTiles[0]);
+        if (group > 0) {
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    parts[(group - 1) * kPart + ((wave * DB + d) * 4 + j) * 64 + lane] =
+                        f32x4{acc[d][4 * j], acc[d][4 * j + 1], acc[d][4 * j + 2], acc[d][4 * j + 3]};
+        }
+        __syncthreads();
+        if (group > 0) return;
+#pragma unroll
+        for (int g = 0; g < G - 1; ++g)
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const f32x4 o = parts[g * kPart + ((wave * DB + d) * 4 + j) * 64 + lane];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[d][4 * j + i] += o[i];
+                }
+    }
     if (!row_ok) return;
     // acc[d][4j + i] is channel 32 d + 8 j + 4 grp + i of this lane's row.
     int8_t *orow = a.out + b * a.o_sb + h * a.o_sh + (int64_t)row * a.o_st;
@@ -415,12 +476,27 @@ extern "C" reef_status reef_attention_int8_integer(
     a.q_tiles = (int32_t)ceil_div(Sq, kIntRows);
     const int64_t items = a.q_tiles * Hq * p->batch;
     if (items >= (int64_t(1) << 31)) return REEF_UNSUPPORTED;
+    // Groups per tile: with few tiles the chain of the heaviest is the time, and two or
+    // four groups halve or quarter it (1x32x2048x128, 512 tiles: 80.5 us with two groups,
+    // 101 with one; one head of 2900 tokens: 87 against 119; head_dim 64, 2x8x1000 over
+    // 1300 keys, 128 tiles: 33.2 with four, 37.5 with two, 55 with one). With more tiles
+    // than two a unit, the units are full without them (4x32x2048x128: 269 with one group,
+    // 316 with two).
     const dim3 grid((unsigned)items);
-    if (D == 128)
-        hipLaunchKernelGGL(int_head_kernel<128>, grid, dim3(kIntThreads), 0, stream, a);
-    else if (D == 64)
-        hipLaunchKernelGGL(int_head_kernel<64>, grid, dim3(kIntThreads), 0, stream, a);
-    else
-        hipLaunchKernelGGL(int_head_kernel<32>, grid, dim3(kIntThreads), 0, stream, a);
+    const int64_t cus = compute_units();
+#define REEF_INT_LAUNCH(DIM, GROUPS)                                                          \
+    hipLaunchKernelGGL((int_head_kernel<DIM, GROUPS>), grid, dim3(GROUPS * kIntThreads), 0, stream, a)
+    if (D == 128) {
+        if (items <= 2 * cus) REEF_INT_LAUNCH(128, 2);
+        else REEF_INT_LAUNCH(128, 1);
+    } else if (D == 64) {
+        if (items <= cus) REEF_INT_LAUNCH(64, 4);
+        else if (items <= 2 * cus) REEF_INT_LAUNCH(64, 2);
+        else REEF_INT_LAUNCH(64, 1);
+    } else {
+        if (items <= cus) REEF_INT_LAUNCH(32, 4);
+        else REEF_INT_LAUNCH(32, 1);
+    }
+#undef REEF_INT_LAUNCH
     return launch_status();
 }

@@ -86,6 +86,32 @@ def test_integer_head_matches_oracle(reef, B, Hq, Hkv, Sq, Skv, D, start, window
             assert np.array_equal(out[b, h], gold), (b, h)
 
 
+@pytest.mark.parametrize("B,H,Sq,Skv,D,window", [
+    (4, 33, 600, 610, 128, 0),    # one group per tile: more than two tiles a compute unit
+    (2, 40, 257, 900, 128, 0),    # two groups, a partial last tile
+    (4, 44, 400, 401, 64, 130),   # one group, a window
+    (3, 30, 400, 530, 64, 0),     # two groups
+    (2, 9, 65, 1, 64, 0),         # four groups, one key tile at most: three have none
+    (1, 5, 190, 500, 64, 100),    # four groups, a window shorter than their stride
+    (3, 30, 400, 420, 32, 0),     # one group
+    (1, 3, 130, 700, 32, 0),      # four groups
+])
+def test_integer_head_groups_bit_exact(reef, B, H, Sq, Skv, D, window):
+    """Every number of groups that the launch chooses by the grid on 256 compute units,
+    with group counts that do not divide the key tiles: the first and the last head."""
+    Skv = max(Skv, Sq)
+    case(f"integer head groups B{B} H{H} Sq{Sq} Skv{Skv} D{D} win{window}")
+    rng = np.random.default_rng(B * 37 + Sq + Skv + D)
+    q = rng.integers(-127, 128, (B, H, Sq, D), dtype=np.int8)
+    k = rng.integers(-127, 128, (B, H, Skv, D), dtype=np.int8)
+    v = rng.integers(-127, 128, (B, H, Skv, D), dtype=np.int8)
+    out = host(reef.attention_int8_integer(gpu(q), gpu(k), gpu(v), table_gpu(), score_shift=10,
+                                           out_shift=8, window=window))
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        gold = oracle.attend_head_int8(q[b, h], k[b, h], v[b, h], Skv - Sq, window, 10, 8)
+        assert np.array_equal(out[b, h], gold), (b, h)
+
+
 def test_integer_head_long_sequence(reef):
     case("integer head 1x1x2048x128 causal, quantized normal data")
     S, D = 2048, 128
