@@ -33,9 +33,11 @@ FLAGS = [
 # Per source: matrix products with their accumulators in ordinary vector registers. Left to
 # itself the compiler moves accumulators between the two register files inside the loops:
 # 120 moves beside 40 products of the GEMM's smaller tiles, and the one-item prefill takes
-# 4 to 7 % longer at head_dim 64 (1x32x2048x64: 47.4 us against 44.2).
+# 4 to 7 % longer at head_dim 64 (1x32x2048x64: 47.4 us against 44.2), the decode over a
+# contiguous cache 2 to 3 % (64 sequences of 100 to 3000 tokens, 16 heads of 64: 94.9 us
+# against 92.2; 64 x 4096, 8 heads of 128: 89 against 87).
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-SOURCE_FLAGS = {"linear.hip": VGPR_FORM, "prefill.hip": VGPR_FORM, "int_head.hip": VGPR_FORM}
+SOURCE_FLAGS = {s: VGPR_FORM for s in ("linear.hip", "prefill.hip", "int_head.hip", "decode.hip")}
 
 
 def commands(objdir):
