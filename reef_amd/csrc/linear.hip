@@ -87,9 +87,9 @@ __device__ __forceinline__ void load_columns(const GemmArgs &a, int n, float (&w
 // half step before is multiplied (two register sets), and the reads and direct loads
 // are issued one by one between the products. Measured (8192 x 8192 -> 8192): 489 us,
 // 2.25 POP/s, where 128 x 128 tiles with two workgroups a unit and no interleaving took
-// 740; 4096 x 8192 -> 6144 in K 4096: 103 against 147; 4096 x 8192 -> 1280: 48.5 against
-// 61.8. Eight waves, two per SIMD, fill each other's waits: 256 x 128 takes 0.97 us a
-// step with eight, 1.07 with four.
+// 740; 4096 x 4096 -> 6144: 103 against 147; 4096 x 8192 -> 1280: 46 against 62. Eight
+// waves, two per SIMD, fill each other's waits: 4096 x 8192 -> 1280 in 256 x 128 tiles
+// takes 50.8 us with eight, 58.2 with four; in 128 x 160 tiles 46 and 48.5.
 //
 // Chunk c (16 bytes) of tile row r sits at chunk_pos in its 128-byte LDS row: the 16
 // lanes that read one chunk of 16 consecutive rows hit 16 distinct bank groups.
@@ -100,10 +100,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, int8_t *smem) {
     constexpr int W = WM * WN;                          // waves, WM x WN over the tile
     constexpr int MI = BM / WM / 16, NJ = BN / WN / 16;  // 16 x 16 blocks per wave
     constexpr int TA = BM * kBK, TB = BN * kBK;         // operand tiles of a stage
-    constexpr int PA = BM / 8 / W, PB = BN / 8 / W;     // 1 KB direct loads per wave
+    constexpr int PA = BM / 8 / W, PB = (BN / 8 + W - 1) / W;  // 1 KB direct loads per wave
     constexpr int kLoads = PA + PB, kFirst = kLoads / 2;
     constexpr int kInFlight = kLoads * (ST - 2);        // loads of the stages after the next
-    static_assert(BM % (8 * W) == 0 && BN % (8 * W) == 0 && W % 2 == 0, "whole loads");
+    static_assert(BM % (8 * W) == 0 && BN % 16 == 0 && W % 2 == 0, "whole loads");
     static_assert(kInFlight + kFirst < 64, "vmcnt fits");
 
     // Workgroup g runs on XCD g % 8: each XCD takes a contiguous run of tiles, in panels
@@ -130,6 +130,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, int8_t *smem) {
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(a.x, xbytes);
     const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(a.w, wbytes);
     uint32_t off[kLoads];
+    // Where the weight tile's blocks do not divide by the waves, a wave without an i-th
+    // block loads its first once more (the same bytes), so that all count the same loads.
+    auto b_block = [&](int i) {
+        return BN / 8 % W == 0 || wave + W * i < BN / 8 ? wave + W * i : wave;
+    };
     // (a wave's blocks are a multiple of 16 rows apart: one chunk position, one k offset)
     const int kch = 16 * chunk_pos(8 * wave + lane / 8, lane % 8);
 #pragma unroll
@@ -139,7 +144,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, int8_t *smem) {
     }
 #pragma unroll
     for (int i = 0; i < PB; ++i) {
-        const int r = n0 + 8 * (wave + W * i) + lane / 8;
+        const int r = n0 + 8 * b_block(i) + lane / 8;
         off[PA + i] = r < a.out ? (uint32_t)((int64_t)r * a.in + kch) : wbytes;
     }
     const int steps = (a.in + kBK - 1) / kBK;
@@ -155,7 +160,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, int8_t *smem) {
                 in_k ? off[i] : xbytes, k0, 0, 0);
         else
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                wr, (__attribute__((address_space(3))) void *)(st + TA + 1024 * W * (i - PA)), 16,
+                wr, (__attribute__((address_space(3))) void *)(st + TA + 1024 * (b_block(i - PA) - wave)), 16,
                 in_k ? off[i] : wbytes, k0, 0, 0);
     };
 
@@ -184,8 +189,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs &a, int8_t *smem) {
     // LDS reads of the next half step's operands and the direct loads [l0, l1) of step s
     // spread between them. Both kinds wait for their place in a queue that the other
     // waves fill as well; issued in one block they kept the matrix core idle for that
-    // time, and a step took the sum of its products, reads and loads (256 x 128, four
-    // waves: 1.09 us a step; loads spread 0.90; both spread 0.84).
+    // time, and a step took the sum of its products, reads and loads (4096 x 8192 -> 1280,
+    // 256 x 128, four waves: 72.6 us; loads spread 62.5; both spread 58.2).
     auto half_step = [&](const Operands &o, Operands &next, const int8_t *st, auto l0_tag,
                          auto l1_tag, int s, int slot) {
         constexpr int l0 = decltype(l0_tag)::value, L = decltype(l1_tag)::value - l0;
@@ -382,7 +387,7 @@ struct TileChoice {
 };
 const TileChoice kTiles[] = {
     {256, 256, 1880, launch_tiles<256, 256, 2, 4, 2>}, {256, 192, 1600, launch_tiles<256, 192, 4, 2, 2>},
-    {256, 128, 970, launch_tiles<256, 128, 4, 2, 3>},  {128, 160, 720, launch_tiles<128, 160, 2, 2, 4>},
+    {256, 128, 970, launch_tiles<256, 128, 4, 2, 3>},  {128, 160, 690, launch_tiles<128, 160, 4, 2, 4>},
     {128, 128, 610, launch_tiles<128, 128, 2, 4, 5>},  {128, 64, 410, launch_tiles<128, 64, 2, 2, 6>},
     {64, 64, 300, launch_tiles<64, 64, 2, 2, 8>},
 };
