@@ -125,7 +125,8 @@ def test_linear_quadrant_tiles(reef, rows, fout, quadrants, monkeypatch):
     (1, 16, 1), (16, 528, 301), (31, 1040, 513),   # 16 features, one or more blocks of 16 rows
     (17, 144, 4001),                               # 16 features, 32 rows
     (16, 272, 6101), (3, 2064, 6100),              # 32 features, 16 rows
-    (100, 400, 2101), (65, 1040, 4160),            # 64 x 64 tiles
+    (100, 400, 2101), (64, 1424, 8170),            # 64 x 32 tiles
+    (65, 1040, 4160),                              # 64 x 64
     (300, 272, 5001),                              # 128 x 64
     (520, 128, 6500),                              # 128 x 128
     (4000, 160, 1270),                             # 128 x 160
