@@ -303,19 +303,23 @@ __global__ __launch_bounds__(64 * W, 1) void gemm_rows_kernel(GemmArgs a) {
     struct Unit {
         i32x4 w[2][NT], x[2][MT];
     };
-    auto load = [&](Unit &u, int k) {  // unit k; chunks past `in` read zeros
+    // Unit k; chunks past `in` read zeros. The range check compares a lane's offset with the
+    // buffer's size less the scalar offset, so that one stays inside a row: the units past
+    // the last and the upper half of a partial one would carry it past the end of a buffer
+    // of one row (only offsets past `in` move: lanes inside it imply k0 <= in - 16).
+    auto load = [&](Unit &u, int k) {
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
-            const int k0 = k * kBK + 64 * half;
+            const int k0 = k * kBK + 64 * half, at = min(k0, a.in - 16);
             const bool in_k = k0 + 16 * grp < a.in;
 #pragma unroll
             for (int j = 0; j < NT; ++j)
                 u.w[half][j] = __builtin_bit_cast(
-                    i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, in_k ? woff[j] : wbytes, k0, 0));
+                    i32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, in_k ? woff[j] : wbytes, at, 0));
 #pragma unroll
             for (int i = 0; i < MT; ++i)
                 u.x[half][i] = __builtin_bit_cast(
-                    i32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, in_k ? xoff[i] : xbytes, k0, 0));
+                    i32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, in_k ? xoff[i] : xbytes, at, 0));
         }
     };
     i32x4 acc[MT][NT];

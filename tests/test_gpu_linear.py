@@ -151,3 +151,23 @@ def test_linear_every_kernel_bit_exact(reef, rows, fin, fout):
     gold = acc * (s[:, None] * ws[None, :]) + b[None, :]
     assert gold.dtype == np.float32
     assert np.array_equal(y.view(np.uint32), gold.view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,fin,fout", [
+    (1, 1040, 1), (1, 1072, 40), (1, 4112, 6144),  # a last unit of 16, 48 and 16 bytes
+    (1, 2128, 1), (5, 3088, 1), (1, 8192, 1280), (2, 1040, 3),
+])
+def test_linear_buffers_of_one_row(reef, rows, fin, fout):
+    """Inputs of one row and weights of one feature in the kernel for few rows, whose loads
+    run up to eight 128-byte units past the end of K: nothing past the row takes part. The
+    weight lies inside a larger tensor of other values."""
+    case(f"w8a8 one row rows{rows} in{fin} out{fout}")
+    rng = np.random.default_rng(rows + fin + fout)
+    x = rng.standard_normal((rows, fin)).astype(np.float32)
+    around = rng.integers(-127, 128, fout * fin + 8192, dtype=np.int8)
+    w = around[4096:4096 + fout * fin].reshape(fout, fin)
+    ws = rng.uniform(0.001, 0.02, fout).astype(np.float32)
+    wt = gpu(around)[4096:4096 + fout * fin].view(fout, fin)
+    y = host(reef.linear_w8a8(gpu(x), wt, gpu(ws)))
+    gold = oracle_linear(x, w, ws)
+    assert np.array_equal(y.view(np.uint32), gold.view(np.uint32))
