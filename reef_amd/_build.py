@@ -37,7 +37,7 @@ FLAGS = [
 # contiguous cache 2 to 3 % (64 sequences of 100 to 3000 tokens, 16 heads of 64: 94.9 us
 # against 92.2; 64 x 4096, 8 heads of 128: 89 against 87).
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-SOURCE_FLAGS = {s: VGPR_FORM for s in ("linear.hip", "prefill.hip", "int_head.hip", "decode.hip")}
+SOURCE_FLAGS = {s: VGPR_FORM for s in ("linear.hip", "prefill.hip", "decode.hip")}
 
 
 def commands(objdir):

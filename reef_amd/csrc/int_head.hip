@@ -82,24 +82,23 @@ struct IntLds {
 // so the groups' results merge exactly through LDS, in any order. The three walks over
 // the keys are one serial chain per tile, which groups shorten (see the launch).
 template <int D, int G>
-__global__ __launch_bounds__(G * kIntThreads, 1) void int_head_kernel(IntHeadArgs a) {
+__global__ __launch_bounds__(G * kIntThreads, G == 1 ? 2 : 1) void int_head_kernel(IntHeadArgs a) {
     using L = IntLds<D>;
     constexpr int DB = D / 32;
-    struct Tiles {
-        int8_t k[2][L::K_BYTES];
-        _Float16 v[2][D * L::V_ROW];
-    };
     __shared__ uint16_t sTable[256];
     __shared__ uint32_t sRow[G][kIntRows];
-    __shared__ __attribute__((aligned(16))) Tiles sTiles[G];
+    // K and V tiles in objects of their own: the compiler then moves reads of one past stores
+    // to the other (in one struct, head_dim 32 takes 1.5 % longer).
+    __shared__ __attribute__((aligned(16))) int8_t sKs[G][2][L::K_BYTES];
+    __shared__ __attribute__((aligned(16))) _Float16 sVs[G][2][D * L::V_ROW];
 
+    const int group = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / kIntThreads);
     const int tid = threadIdx.x & (kIntThreads - 1), lane = tid & 63;
-    const int group = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kIntThreads);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, grp = lane >> 5;
-    auto &sK = sTiles[group].k;
-    auto &sV = sTiles[group].v;
-    if (threadIdx.x < 256) sTable[threadIdx.x] = a.table[threadIdx.x];
+    auto &sK = sKs[group];
+    auto &sV = sVs[group];
+    if (G == 1 || threadIdx.x < 256) sTable[threadIdx.x] = a.table[threadIdx.x];
 
     const int pairs = a.batch * a.q_heads;
     const int tile = a.q_tiles - 1 - (int)blockIdx.x / pairs;  // heaviest first
@@ -185,14 +184,16 @@ __global__ __launch_bounds__(G * kIntThreads, 1) void int_head_kernel(IntHeadArg
     // extra_load(kt) / extra_store(buf) stage more per-tile data the same way.
     auto walk = [&](auto f, auto extra_load, auto extra_store) {
         constexpr int kStep = G * kIntKeys;
-        int kt = kt0 + group * kIntKeys, buf = 0;
-        if (kt <= key_hi) {
-            load_k(kt);
-            extra_load(kt);
+        const int mine = kt0 + group * kIntKeys;
+        if (G == 1 || mine <= key_hi) {
+            load_k(mine);
+            extra_load(mine);
         }
+        int buf = 0;
         // every group runs the same number of barriers
-        for (int first = kt0; first <= key_hi; first += kStep, kt += kStep, buf ^= 1) {
-            if (kt <= key_hi) {
+        for (int first = kt0; first <= key_hi; first += kStep, buf ^= 1) {
+            const int kt = first + group * kIntKeys;
+            if (G == 1 || kt <= key_hi) {
                 store_k(buf);
                 extra_store(buf);
             }
@@ -363,17 +364,23 @@ __global__ __launch_bounds__(G * kIntThreads, 1) void int_head_kernel(IntHeadArg
 
     if constexpr (G > 1) {
         // Groups 1 .. G - 1 leave their products in LDS, lane-linear (conflict-free 16-byte
-        // accesses) over all of the tiles, which the walk's last barrier has freed; group 0
-        // adds them, integers below 2^24 like their sum.
-        constexpr int kPart = 4 * DB * 4 * 64;  // f32x4 per group
-        static_assert((G - 1) * kPart * sizeof(f32x4) <= sizeof(sTiles), "products fit the tiles");
-        f32x4 *parts = reinterpret_cast<f32x4 *>(&sTiles[0]);
+        // accesses) over the V and then the K tiles, which the walk's last barrier has
+        // freed; group 0 adds them, integers below 2^24 like their sum.
+        constexpr int kRuns = 4 * DB * 4;  // runs of 64 f32x4 per group
+        constexpr int kInV = (int)(sizeof(sVs) / (64 * sizeof(f32x4)));
+        constexpr int kInK = (int)(sizeof(sKs) / (64 * sizeof(f32x4)));
+        static_assert((G - 1) * kRuns <= kInV + kInK, "products fit the tiles");
+        auto part = [&](int g, int d, int j) {  // of group g + 1
+            const int r = g * kRuns + (wave * DB + d) * 4 + j;
+            return (r < kInV ? reinterpret_cast<f32x4 *>(&sVs[0][0][0]) + 64 * r
+                             : reinterpret_cast<f32x4 *>(&sKs[0][0][0]) + 64 * (r - kInV)) + lane;
+        };
         if (group > 0) {
 #pragma unroll
             for (int d = 0; d < DB; ++d)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    parts[(group - 1) * kPart + ((wave * DB + d) * 4 + j) * 64 + lane] =
+                    *part(group - 1, d, j) =
                         f32x4{acc[d][4 * j], acc[d][4 * j + 1], acc[d][4 * j + 2], acc[d][4 * j + 3]};
         }
         __syncthreads();
@@ -384,7 +391,7 @@ __global__ __launch_bounds__(G * kIntThreads, 1) void int_head_kernel(IntHeadArg
             for (int d = 0; d < DB; ++d)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const f32x4 o = parts[g * kPart + ((wave * DB + d) * 4 + j) * 64 + lane];
+                    const f32x4 o = *part(g, d, j);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) acc[d][4 * j + i] += o[i];
                 }
@@ -476,22 +483,41 @@ extern "C" reef_status reef_attention_int8_integer(
     a.q_tiles = (int32_t)ceil_div(Sq, kIntRows);
     const int64_t items = a.q_tiles * Hq * p->batch;
     if (items >= (int64_t(1) << 31)) return REEF_UNSUPPORTED;
-    // Groups per tile: with few tiles the chain of the heaviest is the time, and two or
-    // four groups halve or quarter it (1x32x2048x128, 512 tiles: 80.5 us with two groups,
-    // 101 with one; one head of 2900 tokens: 87 against 119; head_dim 64, 2x8x1000 over
-    // 1300 keys, 128 tiles: 33.2 with four, 37.5 with two, 55 with one). With more tiles
-    // than two a unit, the units are full without them (4x32x2048x128: 269 with one group,
-    // 316 with two).
+    // Groups per tile: with at most one tile a compute unit the chain of the heaviest is the
+    // time, and two or four groups shorten it (1x16x2048x128, 256 tiles of up to 32 key
+    // tiles: 68 us with two groups, 91 with one; head_dim 64: 49 with four, 81 with one). With up to two a unit, groups leave no room for a second workgroup
+    // beside the first: a unit then walks its tiles, the launch's n-th and (cus + n)-th
+    // heaviest, one after the other at twice the speed instead of both at once. That gains
+    // where many of them are light (1x32x2048x128, 512 tiles: 78.5 against 96.5; 1x80x512x128:
+    // 26.7 against 30.4) and loses where they weigh alike (queries 512 over 4096 keys, 128
+    // heads of 128: 250 against 221; window 256, 1x32x2048x128: 39.5 against 33; 1x128x512x128:
+    // 36.3 against 32.5). Over 45 shapes each of 288 to 512 tiles, with the key tiles that the
+    // last unit gets, `pair`, and those of the heaviest, two groups take about 1.75 pair + 19
+    // us and one 2.7 heaviest + 11 (head_dim 64: 1.6 pair + 10.5, 2.4 heaviest + 6). With more
+    // tiles than two a unit one group is faster (1024 tiles of 1x64x2048x128: 139 against 158).
     const dim3 grid((unsigned)items);
-    const int64_t cus = compute_units();
+    const int64_t cus = compute_units(), pairs = Hq * p->batch;
+    auto key_tiles = [&](int64_t block) {  // of the block-th workgroup's query tile
+        const int64_t q0 = (a.q_tiles - 1 - block / pairs) * kIntRows;
+        const int64_t lo = p->window > 0 ? std::max<int64_t>(0, p->query_start + q0 + 1 - p->window) : 0;
+        const int64_t hi =
+            std::min(p->query_start + std::min(q0 + kIntRows, Sq) - 1, Skv - 1);
+        return hi / kIntKeys - lo / kIntKeys + 1;
+    };
+    // the last whole tile sees the most keys (a partial one ends earlier)
+    const int64_t heaviest = std::max(key_tiles(0), key_tiles(a.q_tiles > 1 ? pairs : 0));
+    const int64_t pair = items > cus ? key_tiles(cus - 1) + key_tiles(cus) : 0;
+    const bool alone = items <= cus && heaviest > 1, two_a_unit = items > cus && items <= 2 * cus;
 #define REEF_INT_LAUNCH(DIM, GROUPS)                                                          \
     hipLaunchKernelGGL((int_head_kernel<DIM, GROUPS>), grid, dim3(GROUPS * kIntThreads), 0, stream, a)
     if (D == 128) {
-        if (items <= 2 * cus) REEF_INT_LAUNCH(128, 2);
+        if (alone || (two_a_unit && 2 * pair + 10 <= 3 * heaviest)) REEF_INT_LAUNCH(128, 2);
         else REEF_INT_LAUNCH(128, 1);
     } else if (D == 64) {
-        if (items <= cus) REEF_INT_LAUNCH(64, 4);
-        else if (items <= 2 * cus) REEF_INT_LAUNCH(64, 2);
+        // (four groups have work from four key tiles on: 1x128x128x64, two key tiles, 11.8 us
+        // with four, 9.8 with two, 11.0 with one)
+        if (alone && heaviest >= 4) REEF_INT_LAUNCH(64, 4);
+        else if (alone || (two_a_unit && 2 * pair + 6 <= 3 * heaviest)) REEF_INT_LAUNCH(64, 2);
         else REEF_INT_LAUNCH(64, 1);
     } else {
         if (items <= cus) REEF_INT_LAUNCH(32, 4);

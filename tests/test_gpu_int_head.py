@@ -89,12 +89,17 @@ def test_integer_head_matches_oracle(reef, B, Hq, Hkv, Sq, Skv, D, start, window
 @pytest.mark.parametrize("B,H,Sq,Skv,D,window", [
     (4, 33, 600, 610, 128, 0),    # one group per tile: more than two tiles a compute unit
     (2, 40, 257, 900, 128, 0),    # two groups, a partial last tile
+    (2, 40, 500, 500, 128, 0),    # two groups: 320 tiles, many of them light
+    (2, 40, 500, 1900, 128, 0),   # one group: 320 tiles that weigh alike
     (4, 44, 400, 401, 64, 130),   # one group, a window
-    (3, 30, 400, 530, 64, 0),     # two groups
-    (2, 9, 65, 1, 64, 0),         # four groups, one key tile at most: three have none
+    (3, 30, 400, 530, 64, 0),     # one group: 360 tiles that weigh alike
+    (2, 40, 500, 500, 64, 0),     # two groups: 320 tiles, many of them light
+    (2, 9, 65, 1, 64, 0),         # two groups for two key tiles at most
+    (2, 9, 64, 1, 64, 0),         # one group: one key tile
     (1, 5, 190, 500, 64, 100),    # four groups, a window shorter than their stride
     (3, 30, 400, 420, 32, 0),     # one group
     (1, 3, 130, 700, 32, 0),      # four groups
+    (2, 9, 64, 1, 32, 0),         # four groups, one key tile: three have none
 ])
 def test_integer_head_groups_bit_exact(reef, B, H, Sq, Skv, D, window):
     """Every number of groups that the launch chooses by the grid on 256 compute units,
