@@ -153,7 +153,8 @@ __global__ void finalize_scales(float *scales, int64_t n) {
 // ---- per head: x [B, H, S, D] with strides; scale per head over (B, S, D) ---------------
 //
 // The general form, for what the flat form below does not take: head_dim or strides
-// not in whole float4, or strided rows that are not a power of two of float4.
+// not in whole float4, strided rows that are not a power of two of float4, or very many
+// short strided slices.
 // Block (x, h) walks a contiguous range of the head's B * S rows. A row of D values
 // is VEC ? D / 4 float4 : D floats wide; `tpr` threads share a row (all 256 when a
 // row is wider than the block) and 256 / tpr rows are in flight per step, with
@@ -659,14 +660,21 @@ __global__ __launch_bounds__(kQuantThreads) void dequantize(const int8_t *__rest
 
 // The flat kernels over f (q 4-byte aligned, at least 4 * batch * heads * blocks
 // bytes): two launches when the shortest chunk of q holds a head's batch * blocks
-// partial words, three otherwise.
+// partial words, three otherwise. In two, every block writes its partial into the chunks of
+// all blocks of its head; beyond kSpreadWords in all, the stores take longer than a launch
+// (batch 512, 32 heads, 32 tokens of 128: 98 us in three launches, 201 in two with 8 million
+// words; batch 256: 53 against 60; batch 128, half a million words: 31 in either).
+constexpr int64_t kSpreadWords = int64_t(1) << 19;
+
 template <bool NT, bool kRows>
 void launch_flat_as(const FlatHeads &f, int8_t *q, float *scales, uint32_t *status,
                     hipStream_t stream) {
     uint32_t *partials = reinterpret_cast<uint32_t *>(q);
     const dim3 grid((unsigned)f.blocks, (unsigned)f.heads, (unsigned)f.batch);
     const int64_t last4 = f.slice4 - (int64_t)(f.blocks - 1) * f.chunk4;  // shortest chunk
-    if ((int64_t)f.batch * f.blocks <= std::min<int64_t>(last4, 512)) {
+    const int64_t per_head = (int64_t)f.batch * f.blocks;
+    if (per_head <= std::min<int64_t>(last4, 512) &&
+        f.heads * per_head * per_head <= kSpreadWords) {
         hipLaunchKernelGGL((head_max_flat<true, NT, kRows>), grid, dim3(kQuantThreads), 0, stream,
                            f, partials);
         hipLaunchKernelGGL((head_quantize_flat<true, NT, kRows>), grid, dim3(kQuantThreads), 0,
@@ -839,7 +847,14 @@ extern "C" reef_status reef_quantize_int8_per_head(const float *x, int64_t batch
         f.chunk4 = ceil_div(f.slice4, per_slice);
         f.blocks = (int32_t)ceil_div(f.slice4, f.chunk4);
         const int64_t partial_bytes = 4 * batch * heads * (int64_t)f.blocks;
-        if (partial_bytes <= batch * heads * tokens * head_dim && aligned(q, 4)) {
+        // Strided rows stream like consecutive ones unless the slices are many and short: a
+        // block, and a partial, per slice then cost more than the general form's four
+        // launches over all rows (float4 a slice and slices, us flat against general: 32,
+        // 32000, 35 against 18.6; 16, 49152, 52 against 18.7; 128, 32768, 50 against 43; 128,
+        // 16384, 28.1 against 28.3; 256, 32768, 70 against 75; 16, 6144, 12.4 against 13.4).
+        const bool stream_rows =
+            contiguous || batch * heads <= std::max<int64_t>(6144, 128 * f.slice4);
+        if (stream_rows && partial_bytes <= batch * heads * tokens * head_dim && aligned(q, 4)) {
             if (contiguous)
                 launch_flat<false>(f, q, scales, status_word, stream);
             else

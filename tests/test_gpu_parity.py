@@ -165,27 +165,52 @@ def test_quantize_per_head_contiguous_bit_exact(reef, B, H, S, D):
     assert np.array_equal(host(q), qo)
 
 
+def _heads_on_gpu(x, layout):
+    """x [B, H, S, D] on the GPU as itself, as the heads of a projection [B, S, H, D], or as
+    the middle third of a fused one [B, S, 3 H, D]."""
+    if layout == "bhsd":
+        return gpu(x)
+    t = gpu(x.transpose(0, 2, 1, 3))
+    if layout == "qkv":
+        H = x.shape[1]
+        t = torch.cat([t + 1000.0, t, t - 1000.0], dim=2)[:, :, H:2 * H]
+    return t.permute(0, 2, 1, 3)
+
+
 @pytest.mark.parametrize("B,H,S,D", [(1, 3, 31, 128), (1, 8, 33, 128), (2, 5, 64, 128),
                                      (1, 3, 129, 128), (2, 4, 700, 64), (2000, 2, 2, 8),
-                                     (1, 2, 1, 4), (3, 2, 77, 96), (2, 3, 40, 4096)])
-@pytest.mark.parametrize("layout", ["bhsd", "bshd"])
+                                     (1, 2, 1, 4), (3, 2, 77, 96), (2, 3, 40, 4096),
+                                     (1100, 6, 1, 128), (200, 16, 8, 128)])
+@pytest.mark.parametrize("layout", ["bhsd", "bshd", "qkv"])
 def test_quantize_per_head_block_and_rows_bit_exact(reef, layout, B, H, S, D):
     """Heads around the one-block form's limits (1024 and 4096 float4 of a head), then
     the flat streams, with consecutive tokens and with the token stride of a projection;
-    many small batches (the separate scale pass) and rows that are not a power of two."""
+    many small batches (the separate scale pass; strided, the general form from 6144 slices
+    on), more partial words than the two-launch form spreads, and rows that are not a
+    power of two."""
     case(f"quantize_per_head {layout} [{B}, {H}, {S}, {D}]")
     x = W.lcg_normal(29 + S, B * H * S * D).reshape(B, H, S, D)
     x[:, 0] *= 50.0
     x[B - 1, H - 1, S - 1, D - 1] = -300.0  # the last value of the last head decides its scale
-    xt = gpu(x) if layout == "bhsd" else gpu(x.transpose(0, 2, 1, 3)).permute(0, 2, 1, 3)
-    q, s = reef.quantize_per_head(xt)
+    q, s = reef.quantize_per_head(_heads_on_gpu(x, layout))
     qo, so = oracle.quantize_per_head(x)
     assert np.array_equal(host(s).view(np.uint32), so.view(np.uint32))
     assert np.array_equal(host(q), qo)
     x[0, H - 1, 0, 0] = np.inf
-    xt = gpu(x) if layout == "bhsd" else gpu(x.transpose(0, 2, 1, 3)).permute(0, 2, 1, 3)
     with pytest.raises(ValueError):
-        reef.quantize_per_head(xt)
+        reef.quantize_per_head(_heads_on_gpu(x, layout))
+
+
+@pytest.mark.parametrize("B,H,S,D", [(2, 3, 20, 128), (2, 3, 700, 64)])
+def test_quantize_per_head_of_an_expanded_head(reef, B, H, S, D):
+    """One head seen as several (head stride 0): the one-block form and the flat stream."""
+    case(f"quantize_per_head expanded [{B}, {H}, {S}, {D}]")
+    x = W.lcg_normal(47 + S, B * S * D).reshape(B, 1, S, D)
+    xt = gpu(x.transpose(0, 2, 1, 3)).expand(B, S, H, D).permute(0, 2, 1, 3)
+    q, s = reef.quantize_per_head(xt)
+    qo, so = oracle.quantize_per_head(np.ascontiguousarray(np.broadcast_to(x, (B, H, S, D))))
+    assert np.array_equal(host(s).view(np.uint32), so.view(np.uint32))
+    assert np.array_equal(host(q), qo)
 
 
 @pytest.mark.parametrize("rows,width", [(4096, 128), (7, 37), (300, 64), (3, 1), (33, 96),
