@@ -199,8 +199,9 @@ def prefill_kernels(torch, cfg):
     or per-head scales, a workspace): the packed schedule (a V-image pack, then the
     attention kernel) when head_dim is 128 and there is at least one pair of 256-row
     query tiles per compute unit; the balanced schedule with at most one 128-row
-    query tile per compute unit whose heaviest has 18 key tiles more than an equal share;
-    otherwise the split kernel at head_dim 128 and on such small grids, the one-item
+    query tile per compute unit whose heaviest has so many key tiles more than an equal
+    share that cutting it pays (a smaller excess with a tile for almost every unit and a
+    whole number of units per head); otherwise the split kernel at head_dim 128 and on such small grids, the one-item
     kernel at 64. Each is one launch; the packed kernel splits P into fp16
     hi + lo parts for the heads whose values need it, the others always."""
     cus = torch.cuda.get_device_properties(0).multi_processor_count
@@ -211,7 +212,9 @@ def prefill_kernels(torch, cfg):
     items = tiles * cfg.batch * cfg.q_heads
     steps = [(min(128 * (t + 1), cfg.seq) + 63) // 64 for t in range(tiles)]
     share = max(8, sum(steps) * cfg.batch * cfg.q_heads // cus)
-    if items <= cus and max(steps) - share >= 18:
+    even = 16 * items >= 15 * cus and cus % (cfg.batch * cfg.q_heads) == 0
+    line = (11 if even else 20) if cfg.head_dim == 128 else (7 if even else 16)
+    if items <= cus and max(steps) - share >= line:
         return "prefill_stream_kernel"
     return "prefill_split_kernel" if cfg.head_dim == 128 or items <= cus else "prefill_kernel"
 

@@ -924,8 +924,6 @@ constexpr int64_t kQueueWords = 16;  // the last words: the packed schedule's it
 constexpr int64_t kStreamMaxItems = kCounterWords - kQueueWords;
 constexpr int64_t kStreamMinSteps = 8;  // steps per workgroup of the balanced kernels
 constexpr int64_t kStreamCounterBytes = kCounterWords * 4;
-constexpr int64_t kBalanceSteps = 18;  // see the entry point's choice of a schedule
-
 int64_t stream_items(const reef_attention_params &p) {
     return ceil_div(p.q_len, kBM) * p.q_heads * p.batch;
 }
@@ -933,6 +931,36 @@ int64_t stream_items(const reef_attention_params &p) {
 int64_t stream_slot_floats() { return StreamSlot<128>::FLOATS; }
 static_assert(StreamSlot<128>::FLOATS == kPartSlotFloats, "the packed schedule's slots");
 
+
+// Whether the balanced schedule beats the split one on a grid of `items` tiles, at most one
+// per compute unit, the heaviest of `heaviest` key tiles, with equal ranges of `range` of
+// them. The line is the excess of the heaviest over a range; where it lies depends on how
+// many pieces of items the ranges hold. Measured on 329 shapes of each head_dim (us,
+// balanced against split; the excess in brackets):
+//   * every range holds pieces of two items at most, the lightest being no shorter than a
+//     range, as in a chunk over a long prefix: 512 queries over 1536 keys, 8 heads of 128,
+//     35 against 37 (16), 256 over 1280, 64 heads, 35.2 against 34.9 (11); head_dim 64, 25.3
+//     against 28.7 (14), 23.4 against 23.3 (10);
+//   * as many ranges as tiles, a whole number of them for every head: 16 heads of 128, 2048
+//     queries, 44 against 48 (15), 32 heads, 1024 over 2048, 75.8 against 74.8 (7); head_dim
+//     64, 30 against 36 (15), 50.9 against 51.6 (7), 64 heads, 512 over 512, 26.4 against
+//     23.4 (3);
+//   * otherwise light tiles and ends of heads share ranges: 8 heads of 128, 1920 queries, 35
+//     against 44 (22), 1500, 43 against 37 (16), 13 heads, 2048, 52 against 48 (19);
+//     head_dim 64, 8 heads, 1500, 27.6 against 28.4 (16), 1344, 27.9 against 25.4 (13);
+//   * one tile of the same weight for every unit, nothing being cut: 256 heads of 128, 128
+//     queries over 4224 keys, 105 against 111, over 640, 28.7 against 27.5.
+bool balance_pays(const reef_attention_params &p, int64_t items, int64_t heaviest,
+                  int64_t range) {
+    const int64_t cus = compute_units(), tiles = ceil_div(p.q_len, kBM);
+    const int64_t excess = heaviest - range;
+    if (excess == 0 && items == cus) return range >= 32;
+    const bool wide = p.head_dim == 128;
+    if (16 * items >= 15 * cus && cus % (p.batch * p.q_heads) == 0) return excess >= (wide ? 11 : 7);
+    const int64_t lightest = std::min(host_tile_steps(p, 0), host_tile_steps(p, tiles - 1));
+    if (lightest >= range) return excess >= (wide ? 14 : 11);
+    return excess >= (wide ? 20 : 16);
+}
 
 }  // namespace
 }  // namespace reef
@@ -1079,12 +1107,11 @@ extern "C" reef_status reef_attention_prefill_int8(
     }
     // Among the other schedules the library takes
     //   * balanced, which cuts the work of all items into equal ranges, for grids of at
-    //     most one 128-row tile per compute unit whose heaviest tile has kBalanceSteps key
-    //     tiles more than an equal range: that much longer the split kernel would run, at
-    //     1.2 us a key tile (0.8 at head_dim 64), and the cut tiles' merges take about 20 us
-    //     (1x8q/1kv x4096x128, 64 against 33: 61.4 us against 80.3; 1x8x2048x128, 32 against
-    //     8: 35 against 45; 1x8x1024x128, 16 against 8: 31.5 against 27.9; 1x8x200x128, 4
-    //     against 8: 35 against 13.5);
+    //     most one 128-row tile per compute unit whose heaviest tile is enough key tiles
+    //     heavier than an equal range (balance_pays): that much longer the split kernel
+    //     would run, at 1.2 us a key tile (0.8 at head_dim 64), while the pieces of items in
+    //     a range and the merges of cut items take 10 to 30 us (1x8q/1kv x4096x128, 64
+    //     against 33: 61.4 us against 80.3; 1x8x256x128, 4 against 8: 39 against 16);
     //   * split, whose two 4-wave groups halve each tile's key loop, for smaller grids and
     //     at head_dim 128 (1x32x2048x128: 60.5 us against 76.3 one-item; 1x8q/1kv x8192x128:
     //     195 against 278);
@@ -1101,7 +1128,7 @@ extern "C" reef_status reef_attention_prefill_int8(
     const int64_t range = std::max(kStreamMinSteps, per_head * p->batch * Hq / compute_units());
     if (sched == REEF_ATTN_SCHED_BALANCED ||
         (sched == REEF_ATTN_SCHED_AUTO && stream_ok && items <= compute_units() &&
-         (tok || heaviest - range >= kBalanceSteps))) {
+         (tok || balance_pays(*p, items, heaviest, range)))) {
         StreamArgs sa;
         sa.per_head = per_head;
         sa.units = per_head * p->batch * Hq;

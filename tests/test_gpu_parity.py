@@ -438,12 +438,16 @@ def test_prefill_matches_oracle(reef, B, Hq, Hkv, Sq, Skv, D, start, window, gq,
         assert err <= TOL, (precise, sched, ws, err)
 
 
-@pytest.mark.parametrize("S", [1600, 1664])
-@pytest.mark.parametrize("D,start", [(64, 0), (128, 0), (128, 130)])
-def test_prefill_schedule_threshold(reef, S, D, start):
+@pytest.mark.parametrize("D,S,start", [
+    (64, 128, 1024), (64, 128, 1088), (128, 128, 1216), (128, 128, 1280),  # one heavy tile
+    (64, 1472, 0), (64, 1536, 0), (64, 1342, 130), (64, 1406, 130),        # light ones too
+    (128, 1728, 0), (128, 1792, 0), (128, 1598, 130), (128, 1662, 130),
+])
+def test_prefill_schedule_threshold(reef, D, S, start):
     """Grids of at most one tile per compute unit on both sides of the library's line
-    between the split and the balanced schedule (the heaviest of 13 tiles has 25 and 26
-    key tiles against an equal range of 8; with 130 keys before the first row, 27 and 28)."""
+    between the split and the balanced schedule: the heaviest tile has 18 and 19 (head_dim
+    128: 21 and 22) key tiles against an equal range of 8, or, with lighter tiles beside it,
+    23 and 24 (27 and 28)."""
     case(f"prefill schedule threshold S{S} D{D} start{start}")
     B, H = 1, 1
     q = W.lcg_normal(811 + S, B * H * S * D).reshape(B, H, S, D)
@@ -454,6 +458,32 @@ def test_prefill_schedule_threshold(reef, S, D, start):
     err = np.abs(out - gold).max()
     print(f"max_abs_err {err:.3e}", flush=True)
     assert err <= 1e-5  # hi + lo P: 22 bits of weights whose values reach about 4
+
+
+@pytest.mark.parametrize("H,Hkv,S,start", [
+    (256, 2, 128, 1984),  # one tile of the same weight for every unit: nothing is cut
+    (16, 1, 1984, 0),     # as many tiles as ranges, 15 key tiles over a range
+    (64, 4, 500, 500),    # the same, too few over it: split
+])
+def test_prefill_a_tile_for_every_unit(reef, H, Hkv, S, start):
+    """Grids of 256 tiles on both sides of the library's lines: the first and last head."""
+    B, D = 1, 64
+    case(f"prefill a tile for every unit 1x{H}/{Hkv}x{S} over {S + start} keys x64")
+    q = W.lcg_normal(821, B * H * S * D).reshape(B, H, S, D)
+    k = W.lcg_normal(822, B * Hkv * (S + start) * D).reshape(B, Hkv, S + start, D)
+    v = W.lcg_normal(823, B * Hkv * (S + start) * D).reshape(B, Hkv, S + start, D)
+    qo, qs = oracle.quantize_per_head(q)
+    ko, ks = oracle.quantize_per_head(k)
+    vo, vs = oracle.quantize_per_head(v)
+    out = host(reef.attention_prefill(gpu(qo), gpu(ko), gpu(vo), gpu(qs), gpu(ks), gpu(vs)))
+    for h in (0, H - 1):
+        kv = h // (H // Hkv)
+        p = oracle.Problem(1, 1, 1, S, S + start, D, softmax_scale=1 / math.sqrt(D))
+        gold = oracle.attention_int8(p, qo[:, h:h + 1], ko[:, kv:kv + 1], vo[:, kv:kv + 1],
+                                     qs[h:h + 1], ks[kv:kv + 1], vs[kv:kv + 1])
+        err = float(np.abs(out[0, h] - gold[0, 0]).max())
+        print(f"head {h} max_abs_err {err:.3e}", flush=True)
+        assert err <= 1e-5  # as in the test above
 
 
 def test_prefill_outlier_channels(reef):
