@@ -100,8 +100,8 @@ reef_status reef_quantize_int8_per_token(const float *x, int64_t rows, int64_t w
 
 /* The same rows out of a strided [B, H, S, D] tensor (NULL: packed), in [B, H, S]
  * order: q packed [B, H, S, D], scales [B, H, S]. Whole 16-byte rows only (head_dim and
- * strides multiples of 4, x on 16 bytes, head_dim at most 1024): REEF_UNSUPPORTED
- * otherwise. */
+ * strides multiples of 4, x on 16 bytes, head_dim at most 1024) and fewer than 2^31 of
+ * them: REEF_UNSUPPORTED otherwise. */
 reef_status reef_quantize_int8_per_token_heads(const float *x, int64_t batch, int64_t heads,
                                                int64_t tokens, int64_t head_dim,
                                                const reef_strides *x_strides, int8_t *q,

@@ -289,12 +289,15 @@ def quantize_rows(x, status: StatusWord | None = None):
             q = torch.empty(shape, dtype=torch.int8, device=x.device)
             s = torch.empty(shape[:-1], dtype=torch.float32, device=x.device)
             own = status or StatusWord(x.device)
-            check(lib().reef_quantize_int8_per_token_heads(
+            ret = lib().reef_quantize_int8_per_token_heads(
                 _ptr(x), *shape, _STRIDES.pack(sb, sh, st), _ptr(q), _ptr(s), _ptr(own.tensor),
-                _stream()), "quantize_rows")
-            if status is None:
-                own.check("quantize_rows requires finite values")
-            return q, s
+                _stream())
+            if ret != UNSUPPORTED:  # 2^31 rows or more are copied
+                check(ret, "quantize_rows")
+                if status is None:
+                    own.check("quantize_rows requires finite values")
+                return q, s
+            del q, s
     x2 = x if len(shape) == 2 else x.reshape(-1, width)
     if x2.stride(1) != 1:
         x2 = x2.contiguous()

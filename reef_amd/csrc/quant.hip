@@ -924,8 +924,8 @@ extern "C" reef_status reef_quantize_int8_per_token_heads(const float *x, int64_
     if (hr.sb < 0 || hr.sh < 0 || hr.st < 0) return REEF_INVALID_ARGUMENT;
     // whole float4 rows held in a wave's registers, rows counted in 31 bits
     if (head_dim % 4 != 0 || head_dim > 16 * kWave || hr.sb % 4 != 0 || hr.sh % 4 != 0 ||
-        hr.st % 4 != 0 || !aligned(x, 16) || !aligned(q, 4) ||
-        heads >= (int64_t(1) << 31) / tokens || batch >= (int64_t(1) << 31) / (heads * tokens))
+        hr.st % 4 != 0 || !aligned(x, 16) || !aligned(q, 4) || heads > INT32_MAX / tokens ||
+        batch > INT32_MAX / (heads * tokens))
         return REEF_UNSUPPORTED;
     hr.heads = (int32_t)heads;
     hr.tokens = (int32_t)tokens;

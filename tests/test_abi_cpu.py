@@ -177,3 +177,29 @@ def test_integer_head_refuses_rows_beyond_65536_keys():
         rc = lib.reef_attention_int8_integer(C.byref(p), f[0], None, f[1], None, f[2], None, 10,
                                              f[3], 8, f[4], None, None)
         assert rc == reef_amd.UNSUPPORTED
+
+
+@pytest.mark.parametrize("shape", [(1 << 16, 2, 1 << 14, 4), (5, 1 << 28, 3, 8)])
+def test_quantize_rows_of_too_many_strided_heads_copies(monkeypatch, shape):
+    """Strided heads of 2^31 rows or more, which the entry point for heads in place refuses
+    on the host: the wrapper copies them into order first. Tensors without memory; the
+    entry point that would launch is replaced."""
+    torch = pytest.importorskip("torch")
+    lib, calls = reef_amd.lib(), []
+
+    class Lib:
+        reef_quantize_int8_per_token_heads = lib.reef_quantize_int8_per_token_heads
+
+        @staticmethod
+        def reef_quantize_int8_per_token(x, rows, width, stride, *rest):
+            calls.append((rows, width, stride))
+            return reef_amd.OK
+
+    for name, value in (("lib", lambda: Lib), ("_require", lambda *a: None),
+                        ("_ptr", lambda t: 0x10000), ("_stream", lambda: None)):
+        monkeypatch.setattr(reef_amd, name, value)
+    B, S, H, D = shape
+    x = torch.empty((B, S, H, D), device="meta").permute(0, 2, 1, 3)
+    q, scales = reef_amd.quantize_rows(x, status=reef_amd.StatusWord(x.device))
+    assert calls == [(B * H * S, D, D)]
+    assert q.shape == x.shape and q.is_contiguous() and scales.shape == x.shape[:-1]
