@@ -104,58 +104,71 @@ class KvAppendParams(C.Structure):
 
 _P = C.c_void_p
 _I64 = C.c_int64
-_S = C.c_void_p  # a structure: byref(...) or its bytes
+_ST, _AP = C.POINTER(Strides), C.POINTER(AttentionParams)
+_DP, _KP = C.POINTER(DecodeParams), C.POINTER(KvAppendParams)
 _SIGS = {
     "reef_quantize_int8_per_tensor": [_P, _I64, _P, _P, _P, _P],
-    "reef_quantize_int8_per_head": [_P, _I64, _I64, _I64, _I64, _S, _P, _P, _P, _P],
+    "reef_quantize_int8_per_head": [_P, _I64, _I64, _I64, _I64, _ST, _P, _P, _P, _P],
     "reef_quantize_int8_per_token": [_P, _I64, _I64, _I64, _P, _P, _P, _P],
-    "reef_quantize_int8_per_token_heads": [_P, _I64, _I64, _I64, _I64, _S, _P, _P, _P, _P],
+    "reef_quantize_int8_per_token_heads": [_P, _I64, _I64, _I64, _I64, _ST, _P, _P, _P, _P],
     "reef_dequantize_int8": [_P, _I64, _I64, _P, _P, _P],
     "reef_read_status_word": [_P, C.c_int, _P],
-    "reef_attention_prefill_workspace_bytes": [_S],
-    "reef_attention_prefill_int8": [_S, _P, _S, _P, _S, _P, _S, _P, _P, _P, _P, _S, _P,
+    "reef_attention_prefill_workspace_bytes": [_AP],
+    "reef_attention_prefill_int8": [_AP, _P, _ST, _P, _ST, _P, _ST, _P, _P, _P, _P, _ST, _P,
                                     C.c_size_t, _P],
     "reef_qk_scores_i32": [_P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P],
     "reef_qk_scores_i32_packed_workspace_bytes": [_I64, _I64, _I64, _I64, _I64],
     "reef_qk_scores_i32_packed": [_P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, C.c_size_t, _P],
-    "reef_attention_decode_workspace_bytes": [_S],
-    "reef_attention_decode_int8": [_S, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P,
+    "reef_attention_decode_workspace_bytes": [_DP],
+    "reef_attention_decode_int8": [_DP, _P, _P, _P, _P, _P, _P, _P, _P, _P, C.c_size_t, _P,
                                    _P],
-    "reef_attention_decode_int8_paged": [_S, _P, _P, _P, _P, _P, _P, _P,
+    "reef_attention_decode_int8_paged": [_DP, _P, _P, _P, _P, _P, _P, _P,
                                          _I64, _I64, _P, _P, _P, C.c_size_t, _P, _P],
-    "reef_attention_decode_int8_paged_noalloc": [_S, _P, _P, _P, _P, _P, _P,
+    "reef_attention_decode_int8_paged_noalloc": [_DP, _P, _P, _P, _P, _P, _P,
                                                  _P, _I64, _I64, _P, _P, _P, _P],
     "reef_kv_pack_v_pages": [_P, _I64, _I64, _P, _P],
     "reef_linear_w8a8_workspace_bytes": [_I64, _I64],
     "reef_linear_w8a8": [_P, _I64, _I64, _I64, _P, _P, _P, _I64, _P, _I64, _P, C.c_size_t, _P,
                          _P],
     "reef_gemm_w8a8": [_P, _P, _I64, _I64, _P, _P, _P, _I64, _P, _I64, _P, _P],
-    "reef_attention_int8_integer": [_S, _P, _S, _P, _S, _P, _S, C.c_uint32, _P, C.c_uint32, _P,
-                                    _S, _P],
-    "reef_kv_append_int8": [_S, _P, _S, _P, _S, _P, _P, _P, _P, _P, _P, _P, _P],
-    "reef_kv_append_int8_paged": [_S, _P, _S, _P, _S, _P, _P, _I64, _I64, _P, _P, _P, _P, _P, _P,
-                                  _P],
-    "reef_attention_prefill_cache_workspace_bytes": [_S],
-    "reef_attention_prefill_int8_cache": [_S, _P, _S, _P, _P, _P, _P, _P, _I64, _P, _I64, _I64,
-                                          _P, _S, _P, C.c_size_t, _P, _P],
+    "reef_attention_int8_integer": [_AP, _P, _ST, _P, _ST, _P, _ST, C.c_uint32, _P, C.c_uint32,
+                                    _P, _ST, _P],
+    "reef_kv_append_int8": [_KP, _P, _ST, _P, _ST, _P, _P, _P, _P, _P, _P, _P, _P],
+    "reef_kv_append_int8_paged": [_KP, _P, _ST, _P, _ST, _P, _P, _I64, _I64, _P, _P, _P, _P, _P,
+                                  _P, _P],
+    "reef_attention_prefill_cache_workspace_bytes": [_AP],
+    "reef_attention_prefill_int8_cache": [_AP, _P, _ST, _P, _P, _P, _P, _P, _I64, _P, _I64, _I64,
+                                          _P, _ST, _P, C.c_size_t, _P, _P],
 }
 
-_lib_handle = None
+_lib_handle = _plain_handle = None
+
+
+def _load(plain: bool) -> C.CDLL:
+    if not os.path.exists(LIB_PATH):
+        raise RuntimeError(f"{LIB_PATH} is missing: build it with python -m reef_amd._build")
+    handle = C.CDLL(LIB_PATH)
+    for name, args in _SIGS.items():
+        fn = getattr(handle, name)
+        fn.argtypes = [_P if plain and issubclass(t, C._Pointer) else t for t in args]
+        fn.restype = C.c_size_t if name.endswith("_bytes") else C.c_int
+    return handle
 
 
 def lib() -> C.CDLL:
     """The loaded libreef_hip.so. Raises if it has not been built."""
     global _lib_handle
     if _lib_handle is None:
-        if not os.path.exists(LIB_PATH):
-            raise RuntimeError(f"{LIB_PATH} is missing: build it with python -m reef_amd._build")
-        handle = C.CDLL(LIB_PATH)
-        for name, args in _SIGS.items():
-            fn = getattr(handle, name)
-            fn.argtypes = args
-            fn.restype = C.c_size_t if name.endswith("_bytes") else C.c_int
-        _lib_handle = handle
+        _lib_handle = _load(plain=False)
     return _lib_handle
+
+
+def _lib() -> C.CDLL:
+    """The same library with structures as plain addresses, for the wrappers below."""
+    global _plain_handle
+    if _plain_handle is None:
+        _plain_handle = _load(plain=True)
+    return _plain_handle
 
 
 def check(status: int, what: str) -> None:
@@ -238,7 +251,7 @@ class StatusWord:
         return C.c_void_p(self.tensor.data_ptr())
 
     def check(self, what: str) -> None:
-        check(lib().reef_read_status_word(self.ptr, 1, _stream()), what)
+        check(_lib().reef_read_status_word(self.ptr, 1, _stream()), what)
 
 
 # --- quantization (quant.hpp) ---------------------------------------------------------
@@ -251,7 +264,7 @@ def quantize_per_tensor(x, status: StatusWord | None = None):
     q = torch.empty(x.shape, dtype=torch.int8, device=x.device)
     s = torch.empty(1, dtype=torch.float32, device=x.device)
     own = status or StatusWord(x.device)
-    check(lib().reef_quantize_int8_per_tensor(_ptr(x), x.numel(), _ptr(q), _ptr(s), _ptr(own.tensor),
+    check(_lib().reef_quantize_int8_per_tensor(_ptr(x), x.numel(), _ptr(q), _ptr(s), _ptr(own.tensor),
                                               _stream()), "quantize_per_tensor")
     if status is None:
         own.check("quantize_per_tensor requires finite values")
@@ -268,7 +281,7 @@ def quantize_per_head(x, status: StatusWord | None = None):
     q = torch.empty((B, H, S, D), dtype=torch.int8, device=x.device)
     s = torch.empty(H, dtype=torch.float32, device=x.device)
     own = status or StatusWord(x.device)
-    check(lib().reef_quantize_int8_per_head(_ptr(x), B, H, S, D, st, _ptr(q), _ptr(s),
+    check(_lib().reef_quantize_int8_per_head(_ptr(x), B, H, S, D, st, _ptr(q), _ptr(s),
                                             _ptr(own.tensor), _stream()), "quantize_per_head")
     if status is None:
         own.check("quantize_per_head requires finite values")
@@ -289,7 +302,7 @@ def quantize_rows(x, status: StatusWord | None = None):
             q = torch.empty(shape, dtype=torch.int8, device=x.device)
             s = torch.empty(shape[:-1], dtype=torch.float32, device=x.device)
             own = status or StatusWord(x.device)
-            ret = lib().reef_quantize_int8_per_token_heads(
+            ret = _lib().reef_quantize_int8_per_token_heads(
                 _ptr(x), *shape, _STRIDES.pack(sb, sh, st), _ptr(q), _ptr(s), _ptr(own.tensor),
                 _stream())
             if ret != UNSUPPORTED:  # 2^31 rows or more are copied
@@ -305,7 +318,7 @@ def quantize_rows(x, status: StatusWord | None = None):
     q = torch.empty(shape, dtype=torch.int8, device=x.device)
     s = torch.empty(shape[:-1], dtype=torch.float32, device=x.device)
     own = status or StatusWord(x.device)
-    check(lib().reef_quantize_int8_per_token(_ptr(x2), rows, width, x2.stride(0), _ptr(q),
+    check(_lib().reef_quantize_int8_per_token(_ptr(x2), rows, width, x2.stride(0), _ptr(q),
                                              _ptr(s), _ptr(own.tensor), _stream()), "quantize_rows")
     if status is None:
         own.check("quantize_rows requires finite values")
@@ -323,7 +336,7 @@ def dequantize(q, scales, group: int):
     q = q.contiguous()
     x = torch.empty(q.shape, dtype=torch.float32, device=q.device)
     scales = scales.contiguous()
-    check(lib().reef_dequantize_int8(_ptr(q), q.numel(), group, _ptr(scales), _ptr(x),
+    check(_lib().reef_dequantize_int8(_ptr(q), q.numel(), group, _ptr(scales), _ptr(x),
                                      _stream()), "dequantize")
     return x
 
@@ -337,11 +350,11 @@ def prefill_workspace(params: AttentionParams, device):
     """The zero-filled workspace of the balanced prefill schedule, one per (device,
     stream): every launch leaves it zero-filled, so the next launch on that stream
     reuses it."""
-    return _prefill_workspace(C.byref(params), _torch().device(device), _stream())
+    n = lib().reef_attention_prefill_workspace_bytes(C.byref(params))
+    return _prefill_workspace(n, _torch().device(device), _stream())
 
 
-def _prefill_workspace(params, device, stream):
-    n = lib().reef_attention_prefill_workspace_bytes(params)
+def _prefill_workspace(n, device, stream):
     key = (device.index, stream)
     ws = _PREFILL_WS.get(key)
     if ws is None or ws.numel() < n:
@@ -383,13 +396,14 @@ def attention_prefill(q, k, v, q_scales, k_scales, v_scales, *, query_start=None
     qs, ks, vs, os_ = _strides4(q), _strides4(k), _strides4(v), _strides4(out)
     stream = _stream()
     if workspace is None:
-        workspace = _prefill_workspace(p, device, stream)
+        n = _lib().reef_attention_prefill_workspace_bytes(p)
+        workspace = _prefill_workspace(n, device, stream)
     ws_ptr, ws_n = (None, 0) if workspace is False else (_ptr(workspace), workspace.numel()
                                                           * workspace.element_size())
     # (named, so that a copy that contiguous() makes lives until the launch is queued)
     q_scales, k_scales, v_scales = (q_scales.contiguous(), k_scales.contiguous(),
                                     v_scales.contiguous())
-    check(lib().reef_attention_prefill_int8(
+    check(_lib().reef_attention_prefill_int8(
         p, _ptr(q), qs, _ptr(k), ks, _ptr(v), vs, _ptr(q_scales), _ptr(k_scales), _ptr(v_scales),
         _ptr(out), os_, ws_ptr, ws_n, stream), "attention_prefill")
     return out
@@ -419,7 +433,7 @@ def attention_prefill_cache(q, q_scales, k_cache, v_cache, k_scales, v_scales, k
     else:
         max_context, table = 0, block_table.contiguous()
         max_blocks, pages = table.shape[1], k_cache.shape[0]
-    n = lib().reef_attention_prefill_cache_workspace_bytes(p)
+    n = _lib().reef_attention_prefill_cache_workspace_bytes(p)
     device, stream = q.device, _stream()
     key = ("cache", device.index, stream)
     ws = _PREFILL_WS.get(key)
@@ -432,7 +446,7 @@ def attention_prefill_cache(q, q_scales, k_cache, v_cache, k_scales, v_scales, k
     own = status or StatusWord(q.device)
     q_scales, k_cache, v_cache = q_scales.contiguous(), k_cache.contiguous(), v_cache.contiguous()
     k_scales, v_scales = k_scales.contiguous(), v_scales.contiguous()
-    check(lib().reef_attention_prefill_int8_cache(
+    check(_lib().reef_attention_prefill_int8_cache(
         p, _ptr(q), qs, _ptr(q_scales), _ptr(k_cache), _ptr(v_cache), _ptr(k_scales),
         _ptr(v_scales), max_context, _ptr(table), max_blocks, pages, _ptr(out), os_, _ptr(ws), n,
         _ptr(own.tensor), stream), "attention_prefill_cache")
@@ -451,7 +465,7 @@ def qk_scores_i32(q, k):
     B, Hq, Sq, D = q.shape
     Hkv, Skv = k.shape[1], k.shape[2]
     acc = torch.empty((B, Hq, Sq, Skv), dtype=torch.int32, device=q.device)
-    check(lib().reef_qk_scores_i32(_ptr(q), _ptr(k), B, Hq, Hkv, Sq, Skv, D, _ptr(acc),
+    check(_lib().reef_qk_scores_i32(_ptr(q), _ptr(k), B, Hq, Hkv, Sq, Skv, D, _ptr(acc),
                                    _stream()), "qk_scores_i32")
     return acc
 
@@ -469,11 +483,11 @@ def qk_scores_i32_packed(q, k):
     if D != 128:
         raise ValueError("the packed score hook takes head_dim 128")
     acc = torch.full((B, Hq, Sq, Skv), -1, dtype=torch.int32, device=q.device)
-    nbytes = lib().reef_qk_scores_i32_packed_workspace_bytes(B, Hq, Hkv, Sq, Skv)
+    nbytes = _lib().reef_qk_scores_i32_packed_workspace_bytes(B, Hq, Hkv, Sq, Skv)
     if nbytes == 0:
         raise ValueError("qk_scores_i32_packed: invalid sizes")
     ws = torch.zeros(nbytes, dtype=torch.uint8, device=q.device)
-    check(lib().reef_qk_scores_i32_packed(_ptr(q), _ptr(k), B, Hq, Hkv, Sq, Skv, _ptr(acc),
+    check(_lib().reef_qk_scores_i32_packed(_ptr(q), _ptr(k), B, Hq, Hkv, Sq, Skv, _ptr(acc),
                                           _ptr(ws), nbytes, _stream()), "qk_scores_i32_packed")
     return acc
 
@@ -497,12 +511,11 @@ def _decode_params(q, max_context, kv_heads, window, softmax_scale, q_granularit
 def decode_workspace(params: DecodeParams, device):
     """A zero-filled decode workspace (its item counters must start at zero; every
     launch leaves them so, so the workspace is reusable without refilling)."""
-    return _decode_workspace(C.byref(params), device)
+    return _decode_workspace(lib().reef_attention_decode_workspace_bytes(C.byref(params)), device)
 
 
-def _decode_workspace(params, device):
+def _decode_workspace(n, device):
     torch = _torch()
-    n = lib().reef_attention_decode_workspace_bytes(params)
     return torch.zeros(max(n, 16) // 4 + 4, dtype=torch.float32, device=device)
 
 
@@ -521,7 +534,9 @@ def attention_decode(q, q_scales, k_cache, v_pages, k_scales, v_scales, context_
     if tuple(k_cache.shape) != (B, Hkv, L, D) or v_pages.numel() != k_cache.numel():
         raise InvalidArgument("attention_decode cache shape mismatch")
     p = _decode_bytes(q, L, Hkv, window, softmax_scale, q_granularity, num_splits)
-    ws = workspace if workspace is not None else _decode_workspace(p, q.device)
+    ws = workspace
+    if ws is None:
+        ws = _decode_workspace(_lib().reef_attention_decode_workspace_bytes(p), q.device)
     if out is None:
         out = torch.empty((B, Hq, D), dtype=torch.float32, device=q.device)
     own = status or StatusWord(q.device)
@@ -529,7 +544,7 @@ def attention_decode(q, q_scales, k_cache, v_pages, k_scales, v_scales, context_
     q, q_scales, k_cache, v_pages = (q.contiguous(), q_scales.contiguous(), k_cache.contiguous(),
                                      v_pages.contiguous())
     k_scales, v_scales = k_scales.contiguous(), v_scales.contiguous()
-    check(lib().reef_attention_decode_int8(
+    check(_lib().reef_attention_decode_int8(
         p, _ptr(q), _ptr(q_scales), _ptr(k_cache), _ptr(v_pages), _ptr(k_scales), _ptr(v_scales),
         _ptr(cl), _ptr(out), _ptr(ws), ws.numel() * 4, _ptr(own.tensor), _stream()), "attention_decode")
     if status is None:
@@ -550,13 +565,15 @@ def attention_decode_paged(q, q_scales, k_pages, v_pages, k_scale_pages, v_scale
     P, Hkv = k_pages.shape[0], k_pages.shape[1]
     max_blocks = block_table.shape[1]
     p = _decode_bytes(q, max_blocks * PAGE, Hkv, window, softmax_scale, q_granularity, num_splits)
-    ws = workspace if workspace is not None else _decode_workspace(p, q.device)
+    ws = workspace
+    if ws is None:
+        ws = _decode_workspace(_lib().reef_attention_decode_workspace_bytes(p), q.device)
     if out is None:
         out = torch.empty((B, Hq, D), dtype=torch.float32, device=q.device)
     own = status or StatusWord(q.device)
     q, q_scales, block_table, context_lens = (q.contiguous(), q_scales.contiguous(),
                                               block_table.contiguous(), context_lens.contiguous())
-    check(lib().reef_attention_decode_int8_paged(
+    check(_lib().reef_attention_decode_int8_paged(
         p, _ptr(q), _ptr(q_scales), _ptr(k_pages), _ptr(v_pages), _ptr(k_scale_pages),
         _ptr(v_scale_pages), _ptr(block_table), max_blocks, P, _ptr(context_lens), _ptr(out),
         _ptr(ws), ws.numel() * 4, _ptr(own.tensor), _stream()), "attention_decode_paged")
@@ -575,7 +592,7 @@ def pack_v_pages(v_tokens):
     src = v_tokens.contiguous()
     pages = src.numel() // (PAGE * D)
     out = torch.empty((*lead, L // PAGE, D, PAGE), dtype=torch.int8, device=src.device)
-    check(lib().reef_kv_pack_v_pages(_ptr(src), pages, D, _ptr(out), _stream()), "pack_v_pages")
+    check(_lib().reef_kv_pack_v_pages(_ptr(src), pages, D, _ptr(out), _stream()), "pack_v_pages")
     return out
 
 
@@ -605,7 +622,7 @@ def kv_append(k_new, v_new, start_positions, k_cache, v_pages, k_scales, v_scale
     _require(start_positions, torch.int32, "start_positions")
     p = _packed(_APPEND, KvAppendParams, B, H, D, T, L)
     own = status or StatusWord(k_new.device)
-    check(lib().reef_kv_append_int8(
+    check(_lib().reef_kv_append_int8(
         p, _ptr(k_new), ks, _ptr(v_new), vs, _ptr(start_positions),
         _ptr(k_cache), _ptr(v_pages), _ptr(k_scales), _ptr(v_scales), _ptr(context_lens),
         _ptr(own.tensor), _stream()), "kv_append")
@@ -628,7 +645,7 @@ def kv_append_paged(k_new, v_new, start_positions, block_table, k_pages, v_pages
     p = _packed(_APPEND, KvAppendParams, B, H, D, T, max_context or max_blocks * PAGE)
     block_table = block_table.contiguous()
     own = status or StatusWord(k_new.device)
-    check(lib().reef_kv_append_int8_paged(
+    check(_lib().reef_kv_append_int8_paged(
         p, _ptr(k_new), ks, _ptr(v_new), vs, _ptr(start_positions), _ptr(block_table), max_blocks, P, _ptr(k_pages), _ptr(v_pages),
         _ptr(k_scale_pages), _ptr(v_scale_pages), _ptr(context_lens), _ptr(own.tensor), _stream()),
         "kv_append_paged")
@@ -656,7 +673,7 @@ def attention_int8_integer(q, k, v, table, *, score_shift, out_shift=8, query_st
     out = torch.empty((B, Hq, Sq, D), dtype=torch.int8, device=q.device)
     sq, sk, sv, so = _strides4(q), _strides4(k), _strides4(v), _strides4(out)
     table = table.contiguous()
-    check(lib().reef_attention_int8_integer(
+    check(_lib().reef_attention_int8_integer(
         p, _ptr(q), sq, _ptr(k), sk, _ptr(v), sv, score_shift, _ptr(table), out_shift, _ptr(out),
         so, _stream()), "attention_int8_integer")
     return out
@@ -676,13 +693,13 @@ def linear_w8a8(x, weight, w_scales, bias=None, status: StatusWord | None = None
         raise InvalidArgument("linear_w8a8 shapes: x [rows, in], weight [out, in]")
     rows, fin = x.shape
     fout = weight.shape[0]
-    n = lib().reef_linear_w8a8_workspace_bytes(rows, fin)
+    n = _lib().reef_linear_w8a8_workspace_bytes(rows, fin)
     ws = torch.empty(n // 4 + 4, dtype=torch.float32, device=x.device)
     y = torch.empty((rows, fout), dtype=torch.float32, device=x.device)
     own = status or StatusWord(x.device)
     weight, w_scales = weight.contiguous(), w_scales.contiguous()
     bias = bias.contiguous() if bias is not None else None
-    check(lib().reef_linear_w8a8(
+    check(_lib().reef_linear_w8a8(
         _ptr(x), rows, fin, x.stride(0), _ptr(weight), _ptr(w_scales), _ptr(bias), fout, _ptr(y),
         fout, _ptr(ws), ws.numel() * 4, _ptr(own.tensor), _stream()), "linear_w8a8")
     if status is None:

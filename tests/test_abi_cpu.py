@@ -185,7 +185,7 @@ def test_quantize_rows_of_too_many_strided_heads_copies(monkeypatch, shape):
     on the host: the wrapper copies them into order first. Tensors without memory; the
     entry point that would launch is replaced."""
     torch = pytest.importorskip("torch")
-    lib, calls = reef_amd.lib(), []
+    lib, calls = reef_amd._lib(), []
 
     class Lib:
         reef_quantize_int8_per_token_heads = lib.reef_quantize_int8_per_token_heads
@@ -195,7 +195,7 @@ def test_quantize_rows_of_too_many_strided_heads_copies(monkeypatch, shape):
             calls.append((rows, width, stride))
             return reef_amd.OK
 
-    for name, value in (("lib", lambda: Lib), ("_require", lambda *a: None),
+    for name, value in (("_lib", lambda: Lib), ("_require", lambda *a: None),
                         ("_ptr", lambda t: 0x10000), ("_stream", lambda: None)):
         monkeypatch.setattr(reef_amd, name, value)
     B, S, H, D = shape
@@ -203,3 +203,24 @@ def test_quantize_rows_of_too_many_strided_heads_copies(monkeypatch, shape):
     q, scales = reef_amd.quantize_rows(x, status=reef_amd.StatusWord(x.device))
     assert calls == [(B * H * S, D, D)]
     assert q.shape == x.shape and q.is_contiguous() and scales.shape == x.shape[:-1]
+
+
+def test_library_signatures_check_structures():
+    """lib() takes a structure itself or by reference, and refuses another call's structure:
+    read as this call's, its members would mean something else."""
+    lib, p = reef_amd.lib(), good_params()
+    n = lib.reef_attention_prefill_workspace_bytes(C.byref(p))
+    assert n > 0 and lib.reef_attention_prefill_workspace_bytes(p) == n
+    d = DecodeParams(batch=1, q_heads=4, kv_heads=2, head_dim=128, max_context=64, window=0,
+                     softmax_scale=0.1, q_granularity=1, num_splits=0, flags=0)
+    for wrong in (d, C.byref(d)):
+        with pytest.raises(C.ArgumentError):
+            lib.reef_attention_prefill_workspace_bytes(wrong)
+    with pytest.raises(C.ArgumentError):
+        lib.reef_attention_decode_workspace_bytes(C.byref(p))
+    with pytest.raises(C.ArgumentError):
+        reef_amd.decode_workspace(p, "cpu")
+    with pytest.raises(C.ArgumentError):
+        reef_amd.prefill_workspace(d, "cpu")
+    ws = reef_amd.decode_workspace(d, "cpu")
+    assert ws.numel() * 4 >= lib.reef_attention_decode_workspace_bytes(d)
