@@ -135,7 +135,7 @@ __device__ __forceinline__ i32x4 load_stream(const i32x4 *p) {
 
 // One 64-key block in registers: the operands of both matrix products and,
 // per lane, the K and V scale of key 16 grp + col (the 16 lanes of a group
-// hold the 16 scales of its page, handed around with shuffles).
+// hold the 16 scales of its page, handed around within the row).
 template <int D>
 struct DecodeBlock {
     i32x4 k[4][D / 64];
@@ -207,6 +207,16 @@ __device__ __forceinline__ void load_block(const DecodeArgs &a, int b, int kvh, 
     x.vs = gp.vs[col];
 }
 
+// The values of a row's 16 lanes, on every lane of the row (DPP row_newbcast). As shuffles
+// through LDS the 16 index registers made the paged kernel spill inside its key loop (ragged
+// paged decode of 128 sequences: 44.1 us, 41.0 this way).
+template <int R = 0>
+__device__ __forceinline__ void row_lanes(float x, float (&out)[16]) {
+    out[R] = __int_as_float(
+        __builtin_amdgcn_mov_dpp(__float_as_int(x), 0x150 + R, 0xf, 0xf, true));
+    if constexpr (R < 15) row_lanes<R + 1>(x, out);
+}
+
 // Scores, online softmax and P.V of one block for keys [lo, k_end).
 template <int D>
 __device__ __forceinline__ void block_math(const DecodeBlock<D> &cur, int kb, int lo, int k_end,
@@ -216,13 +226,9 @@ __device__ __forceinline__ void block_math(const DecodeBlock<D> &cur, int kb, in
     const int grp = lane >> 4;
     const auto &kop = cur.k;
     const auto &vop = cur.v;
-    const int row0 = lane & ~15;  // first lane of this lane group
     float ksc[16], vsc[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        ksc[r] = __shfl(cur.ks, row0 + r);
-        vsc[r] = __shfl(cur.vs, row0 + r);
-    }
+    row_lanes(cur.ks, ksc);
+    row_lanes(cur.vs, vsc);
     const bool live_g = cur.live;
 
     float x[16];
@@ -291,13 +297,16 @@ __device__ __forceinline__ void block_math(const DecodeBlock<D> &cur, int kb, in
     f16x8 pop[2], plo[2];
     float lp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const float p = __builtin_amdgcn_exp2f(x[r] - m_use);
-        lp[r & 3] += p;
-        const float w = p * (vv[r] * st.inv_s);
-        const _Float16 hi = (_Float16)w;
-        pop[r >> 3][r & 7] = hi;
-        plo[r >> 3][r & 7] = (_Float16)(w - (float)hi);
+    for (int h = 0; h < 2; ++h) {
+        float w[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int r = 8 * h + e;
+            const float p = __builtin_amdgcn_exp2f(x[r] - m_use);
+            lp[r & 3] += p;
+            w[e] = p * (vv[r] * st.inv_s);
+        }
+        split_weights(w, pop[h], plo[h]);
     }
     st.l_run += (lp[0] + lp[1]) + (lp[2] + lp[3]);
     // out^T = V^T . P^T: the output column is the head (lane % 16), the lane

@@ -490,6 +490,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
             for (int u = 0; u < 2; ++u) {
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
+                    float pv[KV_TOKEN ? 8 : 1];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const int r = 8 * s + e;
@@ -506,13 +507,16 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs &a, int tile, int
                                 if (sc[u][r] == INT32_MIN) p = 0.0f;
                             }
                         }
-                        if (KV_TOKEN) l_tile += p;
-                        const float pv =
-                            KV_TOKEN ? p * (sScale[buf][kBN + 32 * u + 16 * grp + r] * inv_s) : p;
-                        const _Float16 hi16 = (_Float16)pv;
-                        phi[u][s][e] = hi16;
-                        plo[u][s][e] = (_Float16)(pv - (float)hi16);
+                        if (KV_TOKEN) {
+                            l_tile += p;
+                            pv[e] = p * (sScale[buf][kBN + 32 * u + 16 * grp + r] * inv_s);
+                        } else {
+                            const _Float16 hi16 = (_Float16)p;
+                            phi[u][s][e] = hi16;
+                            plo[u][s][e] = (_Float16)(p - (float)hi16);
+                        }
                     }
+                    if constexpr (KV_TOKEN) split_weights(pv, phi[u][s], plo[u][s]);
                     if (!KV_TOKEN) {
                         // Row sum of the fp16 probabilities the P.V product uses, two
                         // per instruction, accumulated in fp32.
@@ -773,7 +777,7 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_split_kernel(PrefillA
 }
 
 // Two workgroups share a compute unit, so each SIMD has two waves to fill each other's
-// waits; at head_dim 128 that holds a wave to 256 registers (43 spilled outside the key
+// waits; at head_dim 128 that holds a wave to 256 registers (46 spilled outside the key
 // loop's steady state with per-token scales, 12 without), against 285 and one wave: 4x32/8
 // chunk of 512 over 4096 keys, per token, 207 us against 262; 2x32x2048x128 129 against
 // 167; 1x32x2048x128 per head 61 against 76.

@@ -102,6 +102,19 @@ __device__ __forceinline__ int8_t quantize_int8(float x, float scale) {
     return (int8_t)(int)r;
 }
 
+// Eight weights as fp16, and the fp16 of what that leaves of them: 22 bits together. The
+// empty asm issues nothing; it keeps the rounded weights one value. Without it the compiler
+// converts a weight that is a product twice, for the operand from the rounded product and
+// for the remainder from the unrounded one (v_fma_mixlo_f16, also with contraction off), and
+// where the two round apart, operand and remainder are off by 2^-11 of the weight together.
+__device__ __forceinline__ void split_weights(const float (&w)[8], f16x8 &hi, f16x8 &lo) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) hi[e] = (_Float16)w[e];
+    asm("" : "+v"(hi));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) lo[e] = (_Float16)(w[e] - (float)hi[e]);
+}
+
 __device__ __forceinline__ void flag_status(uint32_t *word, uint32_t bits) {
     if (word) atomicOr(word, bits);
 }

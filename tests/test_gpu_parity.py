@@ -924,6 +924,79 @@ def test_decode_ragged_merge_in_launch(reef, paged, B, Hq, Hkv, D, window, max_l
     assert not host(ws[:B * Hkv]).any()  # the counters lead the workspace
 
 
+def _two_keys(p_first, v, scales):
+    """softmax over two keys in float64: weight of the first, values v [..., 2, D]."""
+    p = p_first[..., None]
+    return p * v[..., 0, :] * scales[..., 0, None] + (1 - p) * v[..., 1, :] * scales[..., 1, None]
+
+
+# Two keys of values up to 4 and per-token scales: an output moves by at most |v0 - v1| / 4
+# <= 2 times the relative error of a weight. Scores stay below 8 in base 2 (three float32
+# roundings, exp2 to 1 ulp: 2.5e-6 of a weight), hi + lo keeps 2^-22 of it, and the sums
+# round at 2^-24 of values of 4: under 6e-6 in all. One weight in some thousand whose parts
+# come from two roundings is off by 2^-11 of itself, about 1e-3.
+TWO_KEYS = 1e-5
+
+
+@pytest.mark.parametrize("D,schedule", [(64, "ONE_ITEM"), (64, "BALANCED"), (128, "ONE_ITEM"),
+                                        (128, "BALANCED")])
+def test_prefill_per_token_weights_are_rounded_once(reef, D, schedule):
+    case(f"prefill per token, window 2, 8x2048x{D} {schedule}")
+    H, S = 8, 2048
+    rng = np.random.default_rng(D)
+    q = rng.integers(-127, 128, (1, H, S, D), dtype=np.int8)
+    k = rng.integers(-127, 128, (1, H, S, D), dtype=np.int8)
+    v = rng.choice(np.array([-127, 127], np.int8), (1, H, S, D))
+    qs = rng.uniform(0.5, 1.0, (1, H, S)).astype(np.float32)
+    ks = rng.uniform(0.5, 1.0, (1, H, S)).astype(np.float32)
+    vs = rng.uniform(0.5, 4.0, (1, H, S)).astype(np.float32) / np.float32(127)
+    scale = 2.0 / (127 * 127 * math.sqrt(D))
+    out = host(reef.attention_prefill(
+        gpu(q), gpu(k), gpu(v), gpu(qs), gpu(ks), gpu(vs), window=2, softmax_scale=scale,
+        q_granularity=reef.PER_TOKEN, kv_granularity=reef.PER_TOKEN,
+        schedule=getattr(reef, f"SCHED_{schedule}")))
+    qd, kd = (t.astype(np.float64) * s[..., None] for t, s in ((q, qs), (k, ks)))
+    own = (qd * kd).sum(-1)[0, :, 1:] * scale           # row i and key i
+    before = (qd[0, :, 1:] * kd[0, :, :-1]).sum(-1) * scale
+    p = 1 / (1 + np.exp(own - before))
+    vd = np.stack([v[0, :, :-1], v[0, :, 1:]], axis=2).astype(np.float64)
+    sd = np.stack([vs[0, :, :-1], vs[0, :, 1:]], axis=2).astype(np.float64)
+    err = np.abs(out[0, :, 1:] - _two_keys(p, vd, sd)).max()
+    print(f"max_abs_err {err:.3e}", flush=True)
+    assert err <= TWO_KEYS
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_weights_are_rounded_once(reef, paged, D):
+    case(f"decode of 2048 sequences of two keys, 16 heads of {D}, paged={paged}")
+    B, H, L = 2048, 16, 16
+    rng = np.random.default_rng(D + 1)
+    q = rng.integers(-127, 128, (B, H, D), dtype=np.int8)
+    k = rng.integers(-127, 128, (B, H, L, D), dtype=np.int8)
+    v = rng.choice(np.array([-127, 127], np.int8), (B, H, L, D))
+    qs = rng.uniform(0.5, 1.0, (B, H)).astype(np.float32)
+    ks = rng.uniform(0.5, 1.0, (B, H, L)).astype(np.float32)
+    vs = rng.uniform(0.5, 4.0, (B, H, L)).astype(np.float32) / np.float32(127)
+    scale = 2.0 / (127 * 127 * math.sqrt(D))
+    lens = gpu(np.full(B, 2, np.int32))
+    vp = reef.pack_v_pages(gpu(v))
+    if paged:  # one page per sequence
+        out = reef.attention_decode_paged(
+            gpu(q), gpu(qs), gpu(k), vp.reshape(B, H, D, L), gpu(ks), gpu(vs),
+            gpu(np.arange(B, dtype=np.int32).reshape(B, 1)), lens, softmax_scale=scale)
+    else:
+        out = reef.attention_decode(gpu(q), gpu(qs), gpu(k), vp, gpu(ks), gpu(vs), lens,
+                                    softmax_scale=scale)
+    s = np.einsum("bhd,bhkd->bhk", q.astype(np.float64) * qs[..., None],
+                  k[:, :, :2].astype(np.float64) * ks[:, :, :2, None]) * scale
+    p = 1 / (1 + np.exp(s[..., 1] - s[..., 0]))
+    err = np.abs(host(out) - _two_keys(p, v[:, :, :2].astype(np.float64),
+                                       vs[:, :, :2].astype(np.float64))).max()
+    print(f"max_abs_err {err:.3e}", flush=True)
+    assert err <= TWO_KEYS
+
+
 def test_decode_paged_flags_bad_pages_and_lengths(reef):
     case("decode paged: out-of-range page and length are reported")
     B, Hq, Hkv, D, lens = 2, 4, 1, 64, [40, 30]
