@@ -134,6 +134,45 @@ def test_append_ties_and_unaligned_rows(reef, D, offset):
     assert np.array_equal(host(dvs).view(np.uint32), vs.view(np.uint32))
 
 
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("paged", [False, True])
+def test_append_writes_lengths_of_their_own(reef, paged, D):
+    """context_lens apart from start_positions, which the append itself then writes, once
+    per sequence: several heads, appends over three and four pages, and a sequence without
+    room, whose length and cache stay."""
+    case(f"kv_append paged={paged} D{D}: lengths of their own, 35 tokens, 5 heads")
+    B, H, L, T = 4, 5, 96, 35
+    starts = np.array([0, 13, 70, 61], np.int32)  # the third would end at 105 > 96
+    k, v, ks, vs = empty_cache(B, H, L, D)
+    kf = W.lcg_normal(31 + D, B * H * T * D).reshape(B, H, T, D)
+    vf = W.lcg_normal(32 + D, B * H * T * D).reshape(B, H, T, D)
+    lens = gpu(np.array([-5, -6, -7, -8], np.int32))
+    if paged:  # page i of sequence b of the cache in pool page table[b, i]
+        n = L // 16
+        table = np.argsort(W.lcg_states(33, B * n), kind="stable").astype(np.int32).reshape(B, n)
+
+        def pages(a):  # [B, H, n, ...] -> pool
+            out = np.empty((B * n,) + a.shape[1:2] + a.shape[3:], a.dtype)
+            out[table.ravel()] = np.moveaxis(a, 2, 1).reshape((B * n,) + out.shape[1:])
+            return out
+        split = lambda: (pages(k.reshape(B, H, n, 16, D)), pages(v),  # noqa: E731
+                         pages(ks.reshape(B, H, n, 16)), pages(vs.reshape(B, H, n, 16)))
+        dev = [gpu(a) for a in split()]
+        call = lambda: reef.kv_append_paged(gpu(kf), gpu(vf), gpu(starts), gpu(table), *dev,  # noqa: E731
+                                            context_lens=lens)
+    else:
+        split = lambda: (k, v, ks, vs)  # noqa: E731
+        dev = [gpu(a) for a in split()]
+        call = lambda: reef.kv_append(gpu(kf), gpu(vf), gpu(starts), *dev, context_lens=lens)  # noqa: E731
+    with pytest.raises(reef.CapacityError):
+        call()
+    for b in (0, 1, 3):
+        expect_rows(k, v, ks, vs, b, int(starts[b]), kf[b], vf[b])
+    for got, want in zip(dev, split()):
+        assert np.array_equal(host(got).view(np.int8), np.ascontiguousarray(want).view(np.int8))
+    assert np.array_equal(host(lens), np.array([35, 48, -7, 96], np.int32))
+
+
 def test_append_capacity_and_non_finite(reef):
     case("kv_append: capacity exceeded for one sequence; non-finite rows")
     B, H, L, D, T = 2, 1, 32, 64, 4

@@ -101,16 +101,11 @@ def test_linear_errors(reef):
 
 
 @pytest.mark.parametrize("rows,fout", [(2000, 2500), (2000, 2980)])
-@pytest.mark.parametrize("quadrants", ["1", "0"])
-def test_linear_quadrant_tiles(reef, rows, fout, quadrants, monkeypatch):
-    """2000 x 256 -> 2500: 16 x 20 = 320 output tiles of 128 x 128, a quarter more
-    than the 256 compute units, so the tiles past the first 256 run as four 64 x 64
-    quadrants each; -> 2980: 16 x 24 = 384 tiles, cut into two 128 x 64 halves. The
-    pieces include the ragged last row and column of tiles. Bit-exact against the
-    oracle with the pieces and with whole tiles only."""
-    monkeypatch.setenv("REEF_GEMM_QUADRANTS", quadrants)
+def test_linear_ragged_output(reef, rows, fout):
+    """2000 x 256 -> 2500 in 128 x 160 tiles and -> 2980 in 256 x 128, one per compute unit
+    or fewer, with a ragged last row and column of tiles. Bit-exact against the oracle."""
     fin = 256
-    case(f"w8a8 rows{rows} in{fin} out{fout} pieces={quadrants}")
+    case(f"w8a8 ragged rows{rows} in{fin} out{fout}")
     rng = np.random.default_rng(77 + fout)
     x = rng.standard_normal((rows, fin)).astype(np.float32)
     w = rng.integers(-127, 128, (fout, fin), dtype=np.int8)
