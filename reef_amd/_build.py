@@ -32,10 +32,11 @@ FLAGS = [
 
 # Per source: matrix products with their accumulators in ordinary vector registers. Left to
 # itself the compiler moves accumulators between the two register files inside the loops:
-# 120 moves beside 40 products of the GEMM's smaller tiles, and the one-item prefill takes
-# 4 to 7 % longer at head_dim 64 (1x32x2048x64: 47.4 us against 44.2), the decode over a
-# contiguous cache 2 to 3 % (64 sequences of 100 to 3000 tokens, 16 heads of 64: 94.9 us
-# against 92.2; 64 x 4096, 8 heads of 128: 89 against 87).
+# 120 moves beside 40 products of the GEMM's smaller tiles (256 x 8192 -> 8192: 41 us with its
+# row quantization, 33.6 this way; 300 x 2048 -> 2048 13.4 against 12.9), the balanced prefill
+# with per-token scales takes 3 to 6 % longer (1x16x1024x128: 40.8 us against 38.5), the
+# decode over a contiguous cache 0.4 % (64 x 4096, 8 heads of 128: 89.6 us against 89.3). The
+# other kernels of prefill.hip and those of int_head.hip come out the same either way.
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 SOURCE_FLAGS = {s: VGPR_FORM for s in ("linear.hip", "prefill.hip", "decode.hip")}
 

@@ -1,13 +1,13 @@
 // W8A8 projection for gfx950: the engine's linear() with a QuantizedWeight
 // (operator/linear.hpp:106-132). Input rows are quantized per row (quantize_rows,
 // quant.hpp:112-133, by the per-token kernel), the int8 rows times the int8
-// weight [out, in] are exact int32 sums on v_mfma_i32_32x32x32_i8, and the
+// weight [out, in] are exact int32 sums on v_mfma_i32_16x16x64_i8, and the
 // epilogue applies y = float(sum) * (row_scale * weight_scale) (+ bias), the
 // engine's float steps in its order, each rounded on its own (no contraction),
 // so the outputs are bit-identical.
 //
-// Two kernels. Many rows: output tiles of BM rows x BN features, one workgroup of 4
-// waves per tile and compute unit, K in 128-byte steps through a ring of LDS stages
+// Two kernels. Many rows: output tiles of BM rows x BN features, one workgroup of four or
+// eight waves per tile and compute unit, K in 128-byte steps through a ring of LDS stages
 // filled by direct-to-LDS buffer loads. Few rows (a decode batch): the weight is read
 // once, straight into the matrix instructions' operand registers, by workgroups that
 // own a few features and split K over their waves.
@@ -82,7 +82,7 @@ __device__ __forceinline__ void load_columns(const GemmArgs &a, int n, float (&w
 // What bounds a tile: its products, and beside them the way of its operands, BM + BN rows
 // through the unit's 64 bytes a cycle from L2 into LDS and from LDS to every wave that
 // needs them (together about the time of the products at 256 x 128). So a workgroup
-// has a compute unit alone, its stages fill the LDS (64 to 128 KB in flight, for an L2 or
+// has a compute unit alone, its stages fill the LDS (112 to 160 KB, for an L2 or
 // memory round trip of several steps), each half step's operands are read while the
 // half step before is multiplied (two register sets), and the reads and direct loads
 // are issued one by one between the products. Measured (8192 x 8192 -> 8192): 489 us,
@@ -384,8 +384,8 @@ void launch_rows_kernel(const GemmArgs &a, hipStream_t stream) {
 // Tiles of BM x BN with WM x WN waves, and the time of one K step (128 bytes) of a
 // workgroup when every compute unit has one, in ns (8192 x 8192 -> 8192 and
 // 4096 x 8192 -> 1280 among others). The larger the tile, the fewer operand bytes per
-// product; the smaller, the more units a small output occupies (64 x 4096 -> 6144: 11.2 us
-// in 192 tiles of 64 x 32, 14.0 in 96 of 64 x 64). A call takes the tile
+// product; the smaller, the more units a small output occupies (64 x 4096 -> 6144: 10.1 us
+// in 192 tiles of 64 x 32, 11.4 in 96 of 64 x 64). A call takes the tile
 // with the least rounds x step time, rounds = ceil(tiles / units).
 struct TileChoice {
     int32_t bm, bn, step_ns;
@@ -418,10 +418,12 @@ reef_status launch_gemm(const int8_t *xq, const float *xs, int64_t rows, int64_t
     const int64_t cus = compute_units();
     // Few rows and features: while 16-feature workgroups with 16 or 32 rows each fit the
     // units at once, every wave's share of K is short and a tile's serial K loop is not
-    // (32 rows, 8192 -> 1280: 9.9 us against 16.3 with 64 x 64 tiles; 64 rows,
-    // 4096 -> 512: 7.3 against 10.7). At most 16 rows take 32 features per workgroup up
-    // to three quarters of the units (16 rows, 4096 -> 6144: 9.4 against 10.9); with
-    // more features the tiles stream the weight as fast.
+    // (32 rows, 8192 -> 1280: 9.9 us against 14.8 in tiles; 64 rows, 4096 -> 512: 6.5
+    // against 9.4). At most 16 rows take 32 features per workgroup up to three quarters of
+    // the units (4 rows, 2048 -> 6144: 5.4 against 6.5; 8 rows, 8192 -> 6144: 13.8 against
+    // 15.1; 16 rows, 4096 -> 6144: 9.1 against 9.3). With more features it is 4 to 6 %
+    // faster at 4096 values a row and 12 % slower at 8192 (-> 8192: 9.0 against 9.6 and 18.0
+    // against 16.0), and past one workgroup a unit slower (4096 -> 11008: 15.2 against 11.3).
     const int64_t nb = ceil_div(out, 16);
     if (ceil_div(rows, 16) * nb <= cus) {
         launch_rows_kernel<1, 1, 8>(a, stream);

@@ -984,8 +984,13 @@ int64_t packed_bytes(const reef_attention_params &p) {
                : 0;
 }
 // The packed schedule is the library's choice for grids with at least one
-// (light, heavy) pair of 256-row query tiles per compute unit; on smaller grids
-// the one-item kernel was measured faster (1x32x2048: 53 against 80 us).
+// (light, heavy) pair of 256-row query tiles per compute unit. Against the one-item kernel
+// it gains with the keys per tile, and where heads take one fp16 P (values within 1) sooner:
+// 4x32x8192 2510 us against 2870 (values to 4), 1770 against 2880 (within 1), 1x32x8192 678
+// against 708, 1x32x4096 232 against 197 and 187 against 196, 2x32x4096 406 against 375 and
+// 320 against 378. Below about 4096 keys the one-item kernel is the faster one by now:
+// 2x32x2048 165 against 111 and 145 against 110, 4x32x1024 137 against 65, 8x32x512 122
+// against 51.
 bool packed_by_default(const reef_attention_params &p) {
     const int64_t pairs = (ceil_div(p.q_len, 256) + 1) / 2 * p.batch * p.q_heads;
     return pairs >= compute_units();
@@ -1116,11 +1121,14 @@ extern "C" reef_status reef_attention_prefill_int8(
     //     would run, at 1.2 us a key tile (0.8 at head_dim 64), while the pieces of items in
     //     a range and the merges of cut items take 10 to 30 us (1x8q/1kv x4096x128, 64
     //     against 33: 61.4 us against 80.3; 1x8x256x128, 4 against 8: 39 against 16);
-    //   * split, whose two 4-wave groups halve each tile's key loop, for smaller grids and
-    //     at head_dim 128 (1x32x2048x128: 60.5 us against 76.3 one-item; 1x8q/1kv x8192x128:
-    //     195 against 278);
+    //   * split, whose two 4-wave groups halve each tile's key loop, for the other small
+    //     grids and at head_dim 128 (1x40x1024x128: 33.2 us against 36.0 one-item; 1x8x8192x128
+    //     181 against 204; but 1x32x2048x128 61.6 against 61.0, 1x64x1024x128 43.5 against
+    //     37.8, 2x24x2048x128 93.7 against 84.6: since the one-item kernel holds two
+    //     workgroups a unit it is the faster one from about 350 tiles on, and this line, with
+    //     packed_by_default's, lies too low for it);
     //   * one-item for larger grids at head_dim 64, where it holds two workgroups a unit
-    //     (1x32x2048x64: 45.8 us against 46.5 split; 4x16x2048x64: 67.8 against 79.8).
+    //     (1x32x2048x64: 43.4 us against 43.3 split; 4x16x2048x64: 66.9 against 80.8).
     // Per-token K/V scales take balanced for at most one tile per unit, one-item otherwise.
     if (sched == REEF_ATTN_SCHED_BALANCED && !stream_ok) return REEF_INVALID_ARGUMENT;
     if (sched == REEF_ATTN_SCHED_SPLIT && tok) return REEF_INVALID_ARGUMENT;
