@@ -171,7 +171,8 @@ reef_status reef_gemm_w8a8(const int8_t *xq, const float *x_scales, int64_t rows
  * pair of 256-row query tiles per compute unit (and a workspace that holds the
  * image); of the others BALANCED, with a large enough workspace, for at most one
  * 128-row query tile per compute unit whose heaviest has many more keys than an equal
- * share (with PER_TOKEN K/V scales for every such grid); otherwise SPLIT for head_dim
+ * share, or whose tiles are equal and fill every unit (with PER_TOKEN K/V scales for
+ * every such grid); otherwise SPLIT for head_dim
  * 128 and for such small grids, ONE_ITEM for head_dim 64 and with PER_TOKEN K/V
  * scales. Every schedule splits P into hi + lo where the values need it. */
 #define REEF_ATTN_SCHED_MASK 0x70u

@@ -779,8 +779,8 @@ __global__ __launch_bounds__(2 * kThreads, 1) void prefill_split_kernel(PrefillA
 // Two workgroups share a compute unit, so each SIMD has two waves to fill each other's
 // waits; at head_dim 128 that holds a wave to 256 registers (46 spilled outside the key
 // loop's steady state with per-token scales, 12 without), against 285 and one wave: 4x32/8
-// chunk of 512 over 4096 keys, per token, 207 us against 262; 2x32x2048x128 129 against
-// 167; 1x32x2048x128 per head 61 against 76.
+// chunk of 512 over 4096 keys, per token, 213 us against 281; 2x32x2048x128 134 against
+// 183; 1x32x2048x128 per head 65 against 83.
 template <int D, bool KV_TOKEN>
 __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(PrefillArgs a) {
     __shared__ __attribute__((aligned(16))) int8_t smem[PrefillLds<D>::BYTES];
