@@ -954,10 +954,9 @@ static_assert(StreamSlot<128>::FLOATS == kPartSlotFloats, "the packed schedule's
 //     head_dim 64, 8 heads, 1500, 27.6 against 28.4 (16), 1344, 27.9 against 25.4 (13);
 //   * one tile of the same weight for every unit, nothing being cut: 256 heads of 128, 128
 //     queries over 4224 keys, 105 against 111, over 640, 28.7 against 27.5.
-bool balance_pays(const reef_attention_params &p, int64_t items, int64_t heaviest,
+bool balance_pays(const reef_attention_params &p, int64_t cus, int64_t items, int64_t heaviest,
                   int64_t range) {
-    const int64_t cus = compute_units(), tiles = ceil_div(p.q_len, kBM);
-    const int64_t excess = heaviest - range;
+    const int64_t tiles = ceil_div(p.q_len, kBM), excess = heaviest - range;
     if (excess == 0 && items == cus) return range >= 32;
     const bool wide = p.head_dim == 128;
     if (16 * items >= 15 * cus && cus % (p.batch * p.q_heads) == 0) return excess >= (wide ? 11 : 7);
@@ -1132,15 +1131,16 @@ extern "C" reef_status reef_attention_prefill_int8(
     // Per-token K/V scales take balanced for at most one tile per unit, one-item otherwise.
     if (sched == REEF_ATTN_SCHED_BALANCED && !stream_ok) return REEF_INVALID_ARGUMENT;
     if (sched == REEF_ATTN_SCHED_SPLIT && tok) return REEF_INVALID_ARGUMENT;
+    const int64_t cus = compute_units();
     const int64_t per_head = host_steps_before(*p, a.q_tiles - 1) +
                              host_tile_steps(*p, a.q_tiles - 1);
     // The last whole tile sees the most keys (a partial one ends earlier).
     const int64_t heaviest = std::max(host_tile_steps(*p, a.q_tiles - 1),
                                       a.q_tiles > 1 ? host_tile_steps(*p, a.q_tiles - 2) : 0);
-    const int64_t range = std::max(kStreamMinSteps, per_head * p->batch * Hq / compute_units());
+    const int64_t range = std::max(kStreamMinSteps, per_head * p->batch * Hq / cus);
     if (sched == REEF_ATTN_SCHED_BALANCED ||
-        (sched == REEF_ATTN_SCHED_AUTO && stream_ok && items <= compute_units() &&
-         (tok || balance_pays(*p, items, heaviest, range)))) {
+        (sched == REEF_ATTN_SCHED_AUTO && stream_ok && items <= cus &&
+         (tok || balance_pays(*p, cus, items, heaviest, range)))) {
         StreamArgs sa;
         sa.per_head = per_head;
         sa.units = per_head * p->batch * Hq;
@@ -1154,7 +1154,7 @@ extern "C" reef_status reef_attention_prefill_int8(
         // workgroup, so that a short chunk of queries over a long prefix is cut into a
         // few parts per item (each merge reads its parts one after another).
         const dim3 sgrid((unsigned)std::min<int64_t>(
-            std::max<int64_t>(1, std::min<int64_t>(compute_units(), sa.units / kStreamMinSteps)),
+            std::max<int64_t>(1, std::min<int64_t>(cus, sa.units / kStreamMinSteps)),
             sa.units));
         // Per-token K/V scales: one 4-wave group per workgroup; otherwise two groups
         // that split each part's key tiles (two waves per SIMD).
@@ -1177,13 +1177,13 @@ extern "C" reef_status reef_attention_prefill_int8(
     }
     const bool split = sched == REEF_ATTN_SCHED_SPLIT ||
                        (sched == REEF_ATTN_SCHED_AUTO && !tok &&
-                        (items <= compute_units() || D == 128));
+                        (items <= cus || D == 128));
     // The 4-wave kernel places two workgroups on each of the 256 compute units at
     // once; zig-zag pairs a heavy and a light tile there. The split kernel holds a
     // compute unit alone and takes the tiles heaviest first.
-    a.zigzag = !split && items <= 2 * compute_units() ? 1 : 0;
+    a.zigzag = !split && items <= 2 * cus ? 1 : 0;
     if (split) {
-        const dim3 pgrid((unsigned)std::min<int64_t>(items, compute_units()));
+        const dim3 pgrid((unsigned)std::min<int64_t>(items, cus));
         if (D == 128)
             hipLaunchKernelGGL(prefill_split_kernel<128>, pgrid, dim3(2 * kThreads), 0, stream, a,
                                (int)items);
